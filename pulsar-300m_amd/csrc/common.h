@@ -215,6 +215,19 @@ __device__ __forceinline__ void lds_barrier() {
 template <typename T>
 constexpr int kVec = 16 / (int)sizeof(T);
 
+// The kVec<T> elements of 16 loaded bytes, to float.
+template <typename T>
+__device__ __forceinline__ void unpackv(const uint4& u, float* o) {
+  if constexpr (sizeof(T) == 2) {
+    unpack_bf16x8(u, o);
+  } else {
+    o[0] = __uint_as_float(u.x);
+    o[1] = __uint_as_float(u.y);
+    o[2] = __uint_as_float(u.z);
+    o[3] = __uint_as_float(u.w);
+  }
+}
+
 __host__ __device__ __forceinline__ bool aligned16(const void* p) {
   return (reinterpret_cast<uintptr_t>(p) & 15u) == 0;
 }
