@@ -182,8 +182,8 @@ def moe_router_topk_forward(logits: torch.Tensor, expert_bias: torch.Tensor, top
     dev = logits.device
     idx = torch.empty((N, top_k), dtype=torch.int64, device=dev)
     w = torch.empty((N, top_k), dtype=torch.bfloat16, device=dev)
-    z = torch.zeros((), dtype=torch.float32, device=dev)
-    pm = torch.zeros(E, dtype=torch.float32, device=dev)
+    z = torch.empty((), dtype=torch.float32, device=dev)
+    pm = torch.empty(E, dtype=torch.float32, device=dev)
     # per-workgroup partial statistics (merged in a fixed order inside the library)
     ws = torch.empty(max(1, _LIB.pulsar_moe_router_workspace_bytes(N, E) // 4),
                      dtype=torch.float32, device=dev)
@@ -270,7 +270,7 @@ def moe_slots_from_order(flat_e: torch.Tensor, order: torch.Tensor, num_experts:
     _req(order.numel() == flat_e.numel(), "order must have as many elements as flat_e")
     M = flat_e.numel()
     slots = torch.empty(M, dtype=torch.int32, device=flat_e.device)
-    counts = torch.zeros(num_experts, dtype=torch.int64, device=flat_e.device)
+    counts = torch.empty(num_experts, dtype=torch.int64, device=flat_e.device)
     order64 = order.to(torch.int64)
     _lib.check(_LIB.pulsar_moe_slots_from_order(_p(flat_e), _p(order64), _p(slots),
                                                 _p(counts), M, num_experts, capacity,
@@ -299,10 +299,10 @@ def rmsnorm_backward(dy: torch.Tensor, x: torch.Tensor, weight: torch.Tensor,
     dim = x.shape[-1]
     rows = x.numel() // dim if dim else 0
     dx = torch.empty_like(x)
-    dw = torch.zeros_like(weight)
     if rows == 0:
-        return [dx, dw]
+        return [dx, torch.zeros_like(weight)]
     _req(dim <= 8192, f"rmsnorm backward supports dim <= 8192, got dim {dim}")
+    dw = torch.empty_like(weight)  # zeroed by the library
     dyc = dy.contiguous()
     rs = rsqrt.float().contiguous()
     _lib.check(_LIB.pulsar_rmsnorm_backward(_p(dyc), _p(x), _p(weight.contiguous()), _p(rs),
@@ -341,7 +341,7 @@ def qk_rmsnorm_rope_backward(dy: torch.Tensor, x: torch.Tensor, weight: torch.Te
             dB, dH, dT = dx.stride(0), dx.stride(1), dx.stride(2)
         else:
             dB, dH, dT = H * T * 64, T * 64, 64
-    dw = torch.zeros_like(weight)
+    dw = torch.empty_like(weight) if n else torch.zeros_like(weight)
     if n:
         cf = cos.float().contiguous()
         sf = sin.float().contiguous()
@@ -383,9 +383,9 @@ def causal_depthwise_conv1d_k4_backward(dout: torch.Tensor, x: torch.Tensor,
     _req(weight.dtype == torch.float32, "weight must be float32")
     B, T, D = x.shape
     dx = torch.empty_like(x)
-    dw = torch.zeros_like(weight)
     if B * T == 0:
-        return [dx, dw]
+        return [dx, torch.zeros_like(weight)]
+    dw = torch.empty_like(weight)  # zeroed by the library
     _lib.check(_LIB.pulsar_causal_conv1d_k4_backward(_p(dout), _p(x), _p(weight), _p(dx), _p(dw),
                                                       B, T, D, code, _stream(x)))
     return [dx, dw]
