@@ -125,6 +125,8 @@ struct GemmArgs {
   int eager_w;
   int a_rows, a_rows0;  // rows of A and A0 (eager_w clamps speculative row indices into them)
   int grid_x, grid_y, grid_z;  // decode bf16 launches: (column block, group, row tile) extents
+  int rows_avg;   // wide launches: expected rows per group (0: max_rows)
+  int rows_fast;  // wide launches of one group: row tiles of a column block follow one another
   int g0_split;  // decode bf16 launches with group 0: grid.y rows of group 0 (its row tiles
                  // spread over g0_split x grid_z workgroups per column block)
 };
@@ -132,9 +134,10 @@ struct GemmArgs {
 int launch_gemm(const GemmArgs& a, int dtype, int epi, int groups, int max_rows,
                 hipStream_t s);
 // Same contract, for row sets of hundreds to tens of thousands of rows (prefill): bf16
-// launches without a fused all-rows group use 128 x 256 output tiles; others fall back to
-// launch_gemm. The two kernels sum K in different orders, so a caller that wants results
-// independent of batch composition picks one by a per-sequence property (prompt length).
+// launches without a fused all-rows group use output tiles of 64 x 64 to 128 x 256, with
+// results that do not depend on the tile; others fall back to launch_gemm. The two kernels
+// sum K in different orders, so a caller that wants results independent of batch composition
+// picks one by a per-sequence property (prompt length).
 int launch_gemm_wide(const GemmArgs& a, int dtype, int epi, int groups, int max_rows,
                      hipStream_t s);
 // Same contract and identical results as launch_gemm (the same summation order), for row

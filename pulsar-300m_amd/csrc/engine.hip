@@ -399,8 +399,8 @@ GemmArgs gemm_base(const Engine& e) {
 }
 
 // Engines whose steps hold kWideHeadRows rows or more (verify blocks, batches of 64+) run
-// the output head in the 128 x 256 LDS tiles of the prefill GEMMs (its 64 MiB of weights
-// read once per 128 rows instead of once per 32); from kWideRows rows (the draft-block
+// the output head in the LDS tiles of the prefill GEMMs (its 64 MiB of weights read once per
+// 128 rows instead of once per 32); from kWideRows rows (the draft-block
 // mode at batch 256) the decode projections too. Below that the row-tile and mid-size
 // GEMMs are faster: 128 x 256 tiles leave most CUs idle at a few hundred rows (320-row
 // verify: 3.78 against 5.35 ms with every projection in wide tiles). The wide tiles sum K
@@ -592,6 +592,7 @@ int enqueue_pass(Engine& e, const StepCtl* ctl, const RowDesc* rows, const AttnU
     g.eager_w = eager_experts;
     g.a_rows = MR;
     g.a_rows0 = MR;
+    g.rows_avg = std::max(1, MR * e.K / e.E);
     if (wide) {
       // wide tiles: the shared expert over all rows, then the routed experts' lists
       GemmArgs gs = gemm_base(e);
@@ -635,6 +636,7 @@ int enqueue_pass(Engine& e, const StepCtl* ctl, const RowDesc* rows, const AttnU
     g.list_count = ra.list_count;
     g.list_stride = lstride;
     g.a_div = 1;
+    g.rows_avg = std::max(1, MR * e.K / e.E);
     g.ctl = ctl;
     if (!wide && (e.ds == e.de || e.ds == 2 * e.de)) {
       g.has_g0 = 1;
@@ -1116,6 +1118,7 @@ int prefill(Engine& e, const int32_t* host_ids, int Bq, int T, hipStream_t s) {
       const int C = (int)std::max<long>(32, ((raw + 31) / 32) * 32);
       // an expert keeps at most C tokens of each sequence
       const int list_max = (int)std::min<long>(BT, (long)Bq * C);
+      const int list_avg = std::max(1, (int)((int64_t)BT * e.K / e.E));
       PULSAR_CHECK_HIP(hipMemsetAsync(e.p_lcount, 0, 4 * (size_t)e.E, s));
       PULSAR_TRY(launch_prefill_capacity(e.topk_idx, e.topk_w, e.keep, e.p_lists, e.p_lcount,
                                          lstride, Bq, T, e.K, e.E, C, s));
@@ -1146,6 +1149,7 @@ int prefill(Engine& e, const int32_t* host_ids, int Bq, int T, hipStream_t s) {
       g.list_count = e.p_lcount;
       g.list_stride = lstride;
       g.a_div = e.K;
+      g.rows_avg = list_avg;
       PULSAR_TRY(gemm_rows(g, EPI_SWIGLU, e.E, list_max));
       g = gemm_base(e);
       g.A = e.act_s;
@@ -1174,6 +1178,7 @@ int prefill(Engine& e, const int32_t* host_ids, int Bq, int T, hipStream_t s) {
       g.list_count = e.p_lcount;
       g.list_stride = lstride;
       g.a_div = 1;
+      g.rows_avg = list_avg;
       g.bias = reinterpret_cast<const char*>(m.routed_scale[l]) + (size_t)k * D * e.es;
       PULSAR_TRY(gemm_rows(g, EPI_SCALE, e.E, list_max));
       CombineArgs ca{};

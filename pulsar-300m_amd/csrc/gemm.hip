@@ -9,18 +9,14 @@
 // expert, all rows, or logits rows), so one launch serves every pulse / expert group and
 // groups without rows exit before touching their weights.
 //
-// Prefill (gemm_bf16_lds_kernel): 128 x 256 output tiles staged through LDS for row sets
-// of thousands of rows, where the work is matrix-core bound rather than weight-bound.
+// Prefill and other wide row sets: gemm_wide.hip.
 //
 // fp32: one wave per output column, lanes split K with 128-bit loads, wave64 reduction.
 #include <algorithm>
 
-#include "engine.h"
+#include "gemm_common.h"
 
 namespace pulsar {
-
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 namespace {
 
@@ -92,96 +88,6 @@ __device__ int resolve_rows(const GemmArgs& g, int group, int tile, int* a_row, 
   return n;
 }
 
-template <typename T>
-__device__ __forceinline__ void epilogue(const GemmArgs& g, int epi, int group, void* Cv,
-                                         int64_t ldc, int crow, int col, float acc, float acc_up) {
-  T* C = reinterpret_cast<T*>(Cv);
-  switch (epi) {
-    case EPI_STORE:
-      C[(int64_t)crow * ldc + col] = from_f<T>(acc);
-      break;
-    case EPI_QKVG:
-      if (col < g.n_main) {
-        C[(int64_t)crow * ldc + col] = from_f<T>(acc);
-      } else {
-        const int h = col - g.n_main;
-        const T* b = reinterpret_cast<const T*>(g.bias) + (int64_t)group * g.bias_group_stride;
-        const float v = rnd<T>(acc + to_f(b[h]));
-        reinterpret_cast<T*>(g.C2)[(int64_t)crow * g.ldc2 + h] = from_f<T>(sigmoidf_(v));
-      }
-      break;
-    case EPI_RESID: {
-      T* p = C + (int64_t)crow * ldc + col;
-      *p = from_f<T>(to_f(*p) + rnd<T>(acc));
-      break;
-    }
-    case EPI_SWIGLU: {
-      const float gt = rnd<T>(acc), up = rnd<T>(acc_up);
-      C[(int64_t)crow * ldc + col] = from_f<T>(gt * sigmoidf_(gt) * up);
-      break;
-    }
-    case EPI_LOGITS: {
-      float l = rnd<T>(acc);
-      if (g.softcap > 0.f) {
-        float t = rnd<T>(l / g.softcap);
-        t = rnd<T>(tanhf(t));
-        l = rnd<T>(g.softcap * t);
-      }
-      reinterpret_cast<float*>(Cv)[(int64_t)crow * ldc + col] = l;
-      break;
-    }
-    case EPI_LOGITS_RAW:
-      reinterpret_cast<float*>(Cv)[(int64_t)crow * ldc + col] = rnd<T>(acc);
-      break;
-    case EPI_SCALE: {
-      const T* s = reinterpret_cast<const T*>(g.bias);
-      C[(int64_t)crow * ldc + col] = from_f<T>(rnd<T>(acc) * to_f(s[col]));
-      break;
-    }
-  }
-}
-
-// Entry i of the group: the row index (pulse / all / logits modes) or the assignment id
-// (list mode; the all-rows group -1 of a fused launch takes row i). Branch-free in the row
-// mode, which is a template parameter: a load pending on one path of a runtime switch
-// would make the join wait for every load in flight, weights included.
-template <int MODE>
-__device__ __forceinline__ int entry_load(const GemmArgs& g, int group, int i) {
-  if constexpr (MODE == ROWS_PULSE) return g.ctl->pulse_start[group] + i;
-  if constexpr (MODE == ROWS_LIST) return g.list[(int64_t)max(group, 0) * g.list_stride + i];
-  return i;
-}
-// Applied after the weight loads are issued (the only use of the loaded value).
-template <int MODE>
-__device__ __forceinline__ int entry_fix(int group, int i, int v) {
-  if constexpr (MODE == ROWS_LIST) return group < 0 ? i : v;
-  return v;
-}
-template <int MODE>
-__device__ __forceinline__ int a_row_of(const GemmArgs& g, int group, int raw) {
-  if constexpr (MODE == ROWS_LIST) {
-    if (group < 0) return raw;
-    // a_div is 1 (expert output rows) or the top-k count (token rows). A power of two takes
-    // a shift instead of the ~30-instruction integer division; entries are non-negative
-    // (only the spare-capacity entries of eager launches may not be, and their rows are
-    // clamped, computed and never stored).
-    const int d = g.a_div;
-    if ((d & (d - 1)) == 0) return raw >> __builtin_ctz((unsigned)d);
-    return raw / d;
-  }
-  return raw;
-}
-template <int MODE>
-__device__ __forceinline__ int group_rows(const GemmArgs& g, int group) {
-  if constexpr (MODE == ROWS_PULSE) return g.ctl->pulse_count[group];
-  if constexpr (MODE == ROWS_LOGITS) return g.ctl->n_lrows;
-  if constexpr (MODE == ROWS_LIST) {
-    // the fused all-rows group (-1) exists only in launches with a step control block
-    return group >= 0 ? g.list_count[group] : g.ctl->n_rows;
-  }
-  return g.ctl ? g.ctl->n_rows : g.m_fixed;
-}
-
 // Workgroup: 16 output columns of one group; 8 waves split K (few registers per wave, so
 // a launch's workgroups are resident at once). The workgroup walks the
 // group's 32-row tiles z, z + gridDim.z, ... keeping its weight slice in registers, so a
@@ -190,7 +96,6 @@ __device__ __forceinline__ int group_rows(const GemmArgs& g, int group) {
 // all-rows group has K0 = KMUL0 * K and runs KMUL0 passes over K-slices (the shared expert
 // down projection fused into the routed one).
 constexpr int kGemmWaves = 8;
-constexpr int kXcds = 8;  // MI355X: consecutive workgroups go to the 8 XCDs in turn
 
 // A launch with several row tiles per group is a 1-D grid over (column block x, group y,
 // row tile z), ordered so that the z workgroups of one (x, y) run one after another on the
@@ -541,252 +446,6 @@ __global__ void __launch_bounds__(256) gemm_f32_kernel(GemmArgs g) {
     s0 = wave_sum(s0);
     if constexpr (kPair) s1 = wave_sum(s1);
     if (lane == (r & 63)) epilogue<float>(g, EPI, group, Cout, ldc, c_row[r], col, s0, s1);
-  }
-}
-
-// Four consecutive output columns of one row (col0 % 4 == 0, never straddling n_main).
-__device__ __forceinline__ void epilogue4(const GemmArgs& g, int epi, int group, void* Cv,
-                                          int64_t ldc, int crow, int col0, const float* v,
-                                          const float* u) {
-  typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
-  bf16* C = reinterpret_cast<bf16*>(Cv);
-  bf16x4_t o;
-  switch (epi) {
-    case EPI_STORE:
-#pragma unroll
-      for (int j = 0; j < 4; ++j) o[j] = (__bf16)v[j];
-      break;
-    case EPI_RESID: {
-      const bf16x4_t h = *reinterpret_cast<const bf16x4_t*>(C + (int64_t)crow * ldc + col0);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) o[j] = (__bf16)((float)h[j] + rnd<bf16>(v[j]));
-      break;
-    }
-    case EPI_SWIGLU:
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float gt = rnd<bf16>(v[j]), up = rnd<bf16>(u[j]);
-        o[j] = (__bf16)(gt * sigmoidf_(gt) * up);
-      }
-      break;
-    case EPI_SCALE: {
-      const bf16x4_t sc = *reinterpret_cast<const bf16x4_t*>(reinterpret_cast<const bf16*>(g.bias) + col0);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) o[j] = (__bf16)(rnd<bf16>(v[j]) * (float)sc[j]);
-      break;
-    }
-    case EPI_LOGITS:
-    case EPI_LOGITS_RAW: {
-      // fp32 store of bf16-rounded logits, softcapped with the scalar epilogue's roundings
-      float4 lv;
-      float* lp = &lv.x;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        float l = rnd<bf16>(v[j]);
-        if (epi == EPI_LOGITS && g.softcap > 0.f) {
-          float t = rnd<bf16>(l / g.softcap);
-          t = rnd<bf16>(tanhf(t));
-          l = rnd<bf16>(g.softcap * t);
-        }
-        lp[j] = l;
-      }
-      *reinterpret_cast<float4*>(reinterpret_cast<float*>(Cv) + (int64_t)crow * ldc + col0) = lv;
-      return;
-    }
-    default:  // EPI_QKVG: q/k/v columns stored, gate columns through the scalar epilogue
-      if (col0 >= g.n_main) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) epilogue<bf16>(g, epi, group, Cv, ldc, crow, col0 + j, v[j], 0.f);
-        return;
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) o[j] = (__bf16)v[j];
-      break;
-  }
-  *reinterpret_cast<bf16x4_t*>(C + (int64_t)crow * ldc + col0) = o;
-}
-
-// LDS-staged tiles for wide row sets: a workgroup of 4 waves owns 128 rows x 256 output
-// columns (SwiGLU: 128 gate columns and their 128 up-projection twins); wave (wr, wc)
-// computes 64 rows x 128 columns as 4 x 8 MFMA tiles (128 accumulators). Per 32-wide k
-// step the workgroup stages the A tile (8 row tiles of 16 rows, gathered rows in MFMA lane
-// order) and 16 weight tiles (1 KB each, stored in lane order) in LDS with direct
-// global-to-LDS loads (16 bytes per lane, no staging registers): a wave's load instruction
-// fills one 1 KB tile, lane l at +16 l, which is the lane's own MFMA operand. A ring of
-// kWideStages buffers keeps kWideStages - 1 k steps in flight while one is computed; one
-// barrier per step both publishes the step's tiles to all waves and frees the buffer the
-// next load overwrites. Each staged byte feeds 2 waves from LDS, and each wave's 12
-// fragment reads feed 32 products. The weights go in as the A operand and the rows as B,
-// so a lane ends with 4 consecutive output columns of its own row: 8-byte epilogue loads
-// and stores, and the C row is an entry the lane loads itself.
-constexpr int kTileRows = 128;
-constexpr int kWideStages = 3;
-
-// Row-set launches of the wide kernel are 1-D grids. The tiles that hold rows, in the order
-// (group, row tile, column block) with column blocks fastest, are cut into 8 equal
-// contiguous ranges, one per XCD (workgroup L runs on XCD L % 8, as slot L / 8 of its
-// range). The column blocks of a row tile then follow one another on one XCD, which
-// fetches the tile's rows into its L2 once for all of them, and a group's weights are read
-// by the one or two XCDs whose ranges hold its tiles. Row counts are read on the device, so
-// every XCD gets an equal share of the tiles that exist; workgroups past the end exit.
-template <int MODE>
-__device__ __forceinline__ bool wide_tile(const GemmArgs& g, int& bx, int& group, int& bz) {
-  const int L = (int)blockIdx.x, xcd = L % kXcds, slot = L / kXcds;
-  const int lane = (int)threadIdx.x & 63;
-  // row tiles of each group, 64 groups per pass (one per lane)
-  int total = 0;
-  for (int y0 = 0; y0 < g.grid_y; y0 += 64) {
-    const int y = y0 + lane;
-    const int nt = y < g.grid_y
-        ? min((group_rows<MODE>(g, y + g.group_offset) + kTileRows - 1) / kTileRows, g.grid_z)
-        : 0;
-    for (int j = 0; j < 64 && y0 + j < g.grid_y; ++j) total += __builtin_amdgcn_readlane(nt, j);
-  }
-  total *= g.grid_x;
-  const int per = (total + kXcds - 1) / kXcds;
-  int item = xcd * per + slot;
-  if (slot >= per || item >= total) return false;
-  bx = item % g.grid_x;
-  int t = item / g.grid_x;
-  for (int y0 = 0; y0 < g.grid_y; y0 += 64) {
-    const int y = y0 + lane;
-    const int nt = y < g.grid_y
-        ? min((group_rows<MODE>(g, y + g.group_offset) + kTileRows - 1) / kTileRows, g.grid_z)
-        : 0;
-    for (int j = 0; j < 64 && y0 + j < g.grid_y; ++j) {
-      const int ntj = __builtin_amdgcn_readlane(nt, j);
-      if (t < ntj) {
-        group = y0 + j + g.group_offset;
-        bz = t;
-        return true;
-      }
-      t -= ntj;
-    }
-  }
-  return false;
-}
-
-template <int EPI, int MODE>
-__global__ void __launch_bounds__(256, 2) gemm_bf16_lds_kernel(GemmArgs g) {
-  constexpr bool kPair = (EPI == EPI_SWIGLU);
-  constexpr int S = kWideStages;
-  __shared__ bf16x8_t sA[S][8][64];   // [buffer][row tile][lane]
-  __shared__ bf16x8_t sW[S][16][64];  // [buffer][column tile][lane]
-  int bx = (int)blockIdx.x, group = (int)blockIdx.y + g.group_offset, bz = (int)blockIdx.z;
-  if constexpr (MODE != ROWS_LOGITS) {
-    if (!wide_tile<MODE>(g, bx, group, bz)) return;
-  }
-  const int N = g.N;
-  const int KT = g.K / 32;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int wr = wv >> 1, wc = wv & 1;
-  const int m16 = lane & 15, kq = lane >> 4;
-  const int cnt = group_rows<MODE>(g, group);
-  if constexpr (MODE == ROWS_LOGITS) {
-    // output head (one group): workgroup L runs on XCD L % 8; give each XCD a contiguous
-    // range of column tiles with their row tiles one after another, so the row tiles of a
-    // column tile read its weights through one L2
-    const int nz = (int)gridDim.z, total = (int)gridDim.x * nz;
-    if (nz > 1 && total % 8 == 0) {
-      const int L = bx + (int)gridDim.x * bz;
-      const int w = (L & 7) * (total >> 3) + (L >> 3);
-      bx = w / nz;
-      bz = w % nz;
-    }
-  }
-  const int r_wg = bz * kTileRows;
-  if (r_wg >= cnt) return;
-  const int ct_wg = bx * (kPair ? 8 : 16);  // first (gate) column tile
-  if (ct_wg * 16 >= N) return;
-  const bf16* A = reinterpret_cast<const bf16*>(g.A);
-  const bf16* W = reinterpret_cast<const bf16*>(g.W) + (int64_t)group * g.w_group_stride;
-
-  // staging: wave wv fills row tiles wv + 4 h (h < 2) and weight tiles wv + 4 h (h < 4).
-  // A row tile's 64 16-byte chunks sit in LDS as (row m, k chunk q) at slot
-  // 4 m + (q ^ (m >> 2 & 3)): the load's lane l carries row 16 t + (l >> 2), so 16 lanes
-  // fetch the 64 contiguous bytes of 4 rows, and the XOR puts the 16 rows of one k chunk
-  // that a fragment read takes on 16 different 16-byte bank groups
-  const bf16* ga[2];
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int r = (wv + 4 * h) * 16 + (lane >> 2);
-    const int i = min(r_wg + r, cnt - 1);
-    const int e = entry_load<MODE>(g, group, i);
-    ga[h] = A + (int64_t)a_row_of<MODE>(g, group, e) * g.lda + ((lane & 3) ^ (lane >> 4 & 3)) * 8;
-  }
-  const int aslot = m16 * 4 + (kq ^ (m16 >> 2 & 3));  // this lane's fragment chunk
-  const bf16* gw[4];
-#pragma unroll
-  for (int h = 0; h < 4; ++h) {
-    const int c = wv + 4 * h;
-    int ct;
-    if constexpr (kPair)
-      ct = c < 8 ? ct_wg + c : N / 16 + ct_wg + (c - 8);
-    else
-      ct = min(ct_wg + c, N / 16 - 1);  // tiles past N re-read the last one (never stored)
-    gw[h] = W + ((int64_t)ct * KT * 64 + lane) * 8;
-  }
-  // k step kt into ring buffer b: 6 loads per wave, counted by vmcnt
-  auto fetch = [&](int kt, int b) {
-#pragma unroll
-    for (int h = 0; h < 4; ++h) load_lds16(gw[h] + (int64_t)kt * 512, &sW[b][wv + 4 * h][0]);
-#pragma unroll
-    for (int h = 0; h < 2; ++h) load_lds16(ga[h] + kt * 32, &sA[b][wv + 4 * h][0]);
-  };
-  // this wave's column tiles in the staged set: 8 of 16 (SwiGLU: 4 gate + their 4 up)
-  int wcol[8];
-#pragma unroll
-  for (int j = 0; j < 8; ++j) wcol[j] = kPair ? (j < 4 ? wc * 4 + j : 8 + wc * 4 + (j - 4)) : wc * 8 + j;
-
-  f32x4_t acc[4][8];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 8; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int k = 0; k < S - 1; ++k)
-    if (k < KT) fetch(k, k);
-  int buf = 0;
-  for (int kt = 0; kt < KT; ++kt) {
-    // this wave's loads of step kt are done once at most the S - 2 younger steps' loads
-    // are outstanding (all of them near the end); the barrier then makes every wave's
-    // tiles of step kt visible and retires step kt - 1, whose buffer the next fetch fills
-    if (kt + S - 2 < KT)
-      wait_vmcnt<6 * (S - 2)>();
-    else
-      wait_vmcnt<0>();
-    lds_barrier();
-    if (kt + S - 1 < KT) fetch(kt + S - 1, buf == 0 ? S - 1 : buf - 1);
-    bf16x8_t fa[4], fw[8];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) fa[i] = sA[buf][wr * 4 + i][aslot];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) fw[j] = sW[buf][wcol[j]][lane];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[j], fa[i], acc[i][j], 0, 0, 0);
-    buf = buf == S - 1 ? 0 : buf + 1;
-  }
-  // lane holds columns 4 kq + e of column tile wcol[j] for row m16 of row tile wr * 4 + i
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = r_wg + wr * 64 + i * 16 + m16;
-    if (r >= cnt) continue;
-    const int crow = entry_fix<MODE>(group, r, entry_load<MODE>(g, group, r)) + g.c_row_offset;
-#pragma unroll
-    for (int j = 0; j < (kPair ? 4 : 8); ++j) {
-      const int col0 = (ct_wg + wcol[j]) * 16 + kq * 4;
-      if (col0 >= N) continue;
-      float v[4], u[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        v[e] = acc[i][j][e];
-        u[e] = kPair ? acc[i][j + 4][e] : 0.f;
-      }
-      epilogue4(g, EPI, group, g.C, g.ldc, crow, col0, v, u);
-    }
   }
 }
 
@@ -1147,56 +806,7 @@ int launch_mid(const GemmArgs& a, int groups, int max_rows, hipStream_t s) {
   return launch_mid_shape<EPI, 1, 4, 6>(a, groups, max_rows, s);
 }
 
-template <int EPI>
-int launch_wide(const GemmArgs& a, int groups, int max_rows, hipStream_t s) {
-  const int colw = EPI == EPI_SWIGLU ? 128 : 256;
-  dim3 grid((unsigned)((a.N + colw - 1) / colw), (unsigned)groups,
-            (unsigned)((max_rows + kTileRows - 1) / kTileRows));
-  // row-set modes: a 1-D grid over (column block, group, row tile), split by wide_tile
-  GemmArgs ga = a;
-  ga.grid_x = (int)grid.x;
-  ga.grid_y = (int)grid.y;
-  ga.grid_z = (int)grid.z;
-  const int64_t tiles = (int64_t)ga.grid_x * ga.grid_y * ga.grid_z;
-  if (tiles > (int64_t)1 << 30) return fail(PULSAR_ERR_INVALID, "gemm: wide launch too large");
-  const dim3 g1((unsigned)((tiles + kXcds - 1) / kXcds * kXcds));
-  switch (a.row_mode) {
-    case ROWS_PULSE: gemm_bf16_lds_kernel<EPI, ROWS_PULSE><<<g1, 256, 0, s>>>(ga); break;
-    case ROWS_LIST: gemm_bf16_lds_kernel<EPI, ROWS_LIST><<<g1, 256, 0, s>>>(ga); break;
-    case ROWS_ALL: gemm_bf16_lds_kernel<EPI, ROWS_ALL><<<g1, 256, 0, s>>>(ga); break;
-    case ROWS_LOGITS:
-      if constexpr (EPI == EPI_LOGITS || EPI == EPI_LOGITS_RAW) {
-        gemm_bf16_lds_kernel<EPI, ROWS_LOGITS><<<grid, 256, 0, s>>>(a);
-        break;
-      }
-      return fail(PULSAR_ERR_INVALID, "gemm: logits rows take a logits epilogue");
-    default: return fail(PULSAR_ERR_INVALID, "gemm: row mode of a wide launch");
-  }
-  PULSAR_LAUNCH_CHECK();
-  return PULSAR_OK;
-}
-
 }  // namespace
-
-int launch_gemm_wide(const GemmArgs& a, int dtype, int epi, int groups, int max_rows,
-                     hipStream_t s) {
-  if (dtype != PULSAR_BF16 || a.has_g0)
-    return launch_gemm(a, dtype, epi, groups, max_rows, s);
-  if (groups <= 0) return PULSAR_OK;
-  if (a.K % 256 != 0 || a.N % 16 != 0 || (epi == EPI_SWIGLU && a.N % 128 != 0))
-    return fail(PULSAR_ERR_UNSUPPORTED, "gemm: wide tiles need K % 256 == 0 and N % 16 == 0 "
-                                        "(SwiGLU: N % 128 == 0)");
-  switch (epi) {
-    case EPI_STORE: return launch_wide<EPI_STORE>(a, groups, max_rows, s);
-    case EPI_QKVG: return launch_wide<EPI_QKVG>(a, groups, max_rows, s);
-    case EPI_RESID: return launch_wide<EPI_RESID>(a, groups, max_rows, s);
-    case EPI_SWIGLU: return launch_wide<EPI_SWIGLU>(a, groups, max_rows, s);
-    case EPI_SCALE: return launch_wide<EPI_SCALE>(a, groups, max_rows, s);
-    case EPI_LOGITS: return launch_wide<EPI_LOGITS>(a, groups, max_rows, s);
-    case EPI_LOGITS_RAW: return launch_wide<EPI_LOGITS_RAW>(a, groups, max_rows, s);
-  }
-  return launch_gemm(a, dtype, epi, groups, max_rows, s);
-}
 
 int launch_gemm_mid(const GemmArgs& a, int dtype, int epi, int groups, int max_rows,
                     hipStream_t s) {
