@@ -56,7 +56,7 @@ struct Engine {
   float* maxprob = nullptr;        // early exit: top-1 probability per logits row
   int32_t* exit_counts = nullptr;  // early exit: [B][4] exits per pulse
   int32_t *lists = nullptr, *list_count = nullptr;      // decode: [L][E][max_rows*K], [L][E]
-  int32_t *p_lists = nullptr, *p_lcount = nullptr;  // prefill
+  int32_t *p_lists = nullptr, *p_lcount = nullptr;  // prefill (counts per pulse and layer)
   int32_t* p_ids = nullptr;
   RowDesc* p_rows = nullptr;  // [P][R]
   StepCtl* p_ctl = nullptr;   // [P]
@@ -339,7 +339,7 @@ int create(const PulsarModelDesc& m, const PulsarEngineConfig& c, Engine** out) 
   PULSAR_TRY(x.alloc(&x.lists, 4 * (size_t)x.L * x.E * MR * x.K));
   PULSAR_TRY(x.alloc(&x.list_count, 4 * (size_t)x.L * x.E));
   PULSAR_TRY(x.alloc(&x.p_lists, 4 * (size_t)x.E * R * x.K));
-  PULSAR_TRY(x.alloc(&x.p_lcount, 4 * (size_t)x.E));
+  PULSAR_TRY(x.alloc(&x.p_lcount, 4 * (size_t)x.E * x.L * x.P));
   PULSAR_TRY(x.alloc(&x.p_ids, 4 * (size_t)x.B * c.max_prompt));
   PULSAR_TRY(x.alloc(&x.p_rows, sizeof(RowDesc) * x.P * (size_t)x.B * c.max_prompt));
   PULSAR_TRY(x.alloc(&x.p_ctl, sizeof(StepCtl) * x.P));
@@ -979,6 +979,8 @@ int prefill(Engine& e, const int32_t* host_ids, int Bq, int T, hipStream_t s) {
   PULSAR_CHECK_HIP(hipMemcpyAsync(e.p_ctl, ctls.data(), sizeof(StepCtl) * P,
                                   hipMemcpyHostToDevice, s));
   PULSAR_CHECK_HIP(hipMemsetAsync(e.ctl, 0, sizeof(StepCtl), s));
+  // kept rows per expert of every (pulse, layer)
+  PULSAR_CHECK_HIP(hipMemsetAsync(e.p_lcount, 0, 4 * (size_t)e.E * e.L * e.P, s));
 
   PULSAR_TRY(launch_prefill_stem(e.p_ids, m.tok_emb, m.anchor_norm, m.conv_w, e.xn, e.e_state,
                                  Bq, T, D, m.rms_eps, dt, s));
@@ -1119,8 +1121,8 @@ int prefill(Engine& e, const int32_t* host_ids, int Bq, int T, hipStream_t s) {
       // an expert keeps at most C tokens of each sequence
       const int list_max = (int)std::min<long>(BT, (long)Bq * C);
       const int list_avg = std::max(1, (int)((int64_t)BT * e.K / e.E));
-      PULSAR_CHECK_HIP(hipMemsetAsync(e.p_lcount, 0, 4 * (size_t)e.E, s));
-      PULSAR_TRY(launch_prefill_capacity(e.topk_idx, e.topk_w, e.keep, e.p_lists, e.p_lcount,
+      int32_t* lcount = e.p_lcount + (size_t)(k * e.L + l) * e.E;
+      PULSAR_TRY(launch_prefill_capacity(e.topk_idx, e.topk_w, e.keep, e.p_lists, lcount,
                                          lstride, Bq, T, e.K, e.E, C, s));
       g = gemm_base(e);
       g.A = e.xn;
@@ -1146,7 +1148,7 @@ int prefill(Engine& e, const int32_t* host_ids, int Bq, int T, hipStream_t s) {
       g.N = e.de;
       g.row_mode = ROWS_LIST;
       g.list = e.p_lists;
-      g.list_count = e.p_lcount;
+      g.list_count = lcount;
       g.list_stride = lstride;
       g.a_div = e.K;
       g.rows_avg = list_avg;
@@ -1175,7 +1177,7 @@ int prefill(Engine& e, const int32_t* host_ids, int Bq, int T, hipStream_t s) {
       g.N = D;
       g.row_mode = ROWS_LIST;
       g.list = e.p_lists;
-      g.list_count = e.p_lcount;
+      g.list_count = lcount;
       g.list_stride = lstride;
       g.a_div = 1;
       g.rows_avg = list_avg;

@@ -6,6 +6,8 @@
 // Rounding follows the reference op by op: every intermediate the reference materialises
 // in the activation dtype T is rounded through T here (rnd<T>), so fp32 runs differ from
 // the reference only by summation order and bf16 runs see the same quantisation points.
+#include <type_traits>
+
 #include "rows.h"
 
 namespace pulsar {
@@ -1329,9 +1331,9 @@ __global__ void __launch_bounds__(256) attn_prefill_kernel(AttnArgs a) {
 
 // ---------------------------------------------------------------------------
 // Prefill attention in bf16 on the matrix cores (same key ranges as attn_prefill_kernel).
-// Block = (sequence, 64-query tile, kv head); wave w takes query head 4g + w % 4 over
-// 16·NQ of the tile's 64 queries, so each 64-key block staged in LDS serves every head and
-// query of the block. Per block:
+// Block = (sequence, tile of 16 NQ NG queries, kv head); wave w takes query head 4g + w % 4
+// over the tile's w / 4-th group of 16 NQ queries, so each 64-key block staged in LDS serves
+// every head and query of the block. Per block:
 // S^T = K Q^T (keys x queries), online softmax per query, O^T += V^T P^T (dims x queries).
 // In this orientation P never leaves the registers: the D tile of S^T gives lane l keys
 // 4*(l/16) + j (j < 4) of query l % 16, and the B operand of the second product takes 8
@@ -1339,26 +1341,26 @@ __global__ void __launch_bounds__(256) attn_prefill_kernel(AttnArgs a) {
 // permutation of the reduction index that the V^T operand repeats (V^T is staged with those
 // 8 keys in consecutive slots: one 16-byte LDS read per fragment).
 // Scores use exp2 with log2(e) folded into the scale; P is rounded to bf16 for the second
-// product, the running max, sum and output accumulate in fp32.
+// product, the running maximum, sum and output accumulate in fp32. A query's arithmetic is
+// the same in every tile size.
+// Two LDS buffers (one barrier per block), and the next one or two blocks in flight in registers.
 // ---------------------------------------------------------------------------
 
-// At least 4 waves per SIMD (at most 128 registers per lane): with NQ = 2 two workgroups of
-// 8 waves share a CU, so one computes while the other waits at its barriers.
-template <int NQ>
-__global__ void __launch_bounds__(256 * (4 / NQ), 4) attn_prefill_mfma_kernel(AttnArgs a) {
-  // NQ 16-query tiles per wave: the 64 queries of the block are split over 4 / NQ waves
-  // per head, so the block has 4 heads x (4 / NQ) waves
-  constexpr int kThreads = 256 * (4 / NQ);
-  // 16-byte chunks of each staged tile per staging thread (the first 512 threads stage)
-  constexpr int CH = kThreads >= 512 ? 1 : 512 / kThreads;
-  const bool stager = threadIdx.x < 512;
+// At least 4 waves per SIMD (at most 128 registers per lane): two workgroups of 8 waves share
+// a CU, so one computes while the other waits at its barriers.
+template <int NQ, int NG>
+__global__ void __launch_bounds__(256 * NG, NG == 1 ? 2 : 4) attn_prefill_mfma_kernel(AttnArgs a) {
+  constexpr int kThreads = 256 * NG, kQ = 16 * NQ * NG;
+  constexpr int CH = 512 / kThreads;  // 16-byte chunks of each staged tile per thread
+  static_assert(NG == 1 || NG == 2, "256 or 512 threads");
+  constexpr int PF = NG == 1 ? 2 : 1;  // blocks in flight (two at 8 waves spill)
   constexpr int kLd = 72;  // LDS row stride in bf16: 16 bytes of padding against bank conflicts
-  __shared__ __attribute__((aligned(16))) __bf16 Ks[64][kLd];  // [key][dim]
+  __shared__ __attribute__((aligned(16))) __bf16 Ks[2][64][kLd];  // [buffer][key][dim]
   // [dim][key slot]: within each 32-key half, lane kq's 8 keys of the second product (keys
   // 4 kq .. 4 kq + 3 of both 16-key tiles) sit in slots 8 kq .. 8 kq + 7
-  __shared__ __attribute__((aligned(16))) __bf16 Vs[64][kLd];
+  __shared__ __attribute__((aligned(16))) __bf16 Vs[2][64][kLd];
   const int T_ = a.prefill_T;
-  const int ntile = (T_ + 63) / 64;
+  const int ntile = (T_ + kQ - 1) / kQ;
   const int b = (int)blockIdx.x / ntile;
   const int qt = ntile - 1 - (int)blockIdx.x % ntile;  // longest key ranges first
   const int g = blockIdx.y;
@@ -1367,8 +1369,8 @@ __global__ void __launch_bounds__(256 * (4 / NQ), 4) attn_prefill_mfma_kernel(At
   const int head = g * 4 + (wv & 3);
   const int qoff = (wv >> 2) * 16 * NQ;  // this wave's first query within the block
   const bool quirk = a.is_local && T_ > a.window;
-  const int q0 = qt * 64;
-  const int qlast = min(q0 + 63, T_ - 1);
+  const int q0 = qt * kQ;
+  const int qlast = min(q0 + kQ - 1, T_ - 1);
   const int tlo = quirk ? T_ - a.window : 0;
   const int thi = quirk ? T_ - a.window + min(qlast, a.window - 1) : qlast;
   // keys every query of the tile sees: blocks inside [flo, fhi] need no mask
@@ -1400,46 +1402,42 @@ __global__ void __launch_bounds__(256 * (4 / NQ), 4) attn_prefill_mfma_kernel(At
   const float sl2 = a.scale * 1.4426950408889634f;
 
   // staging: thread -> CH 16-byte chunks of K row sr (dims from sc) and of V row sr (keys)
-  const int sr = ((tid & 511) * CH) >> 3, sc16 = (((tid & 511) * CH) & 7) * 8;
+  const int sr = (tid * CH) >> 3, sc16 = ((tid * CH) & 7) * 8;
   const bf16* Kc = reinterpret_cast<const bf16*>(a.kv.k[a.layer]);
   const bf16* Vc = reinterpret_cast<const bf16*>(a.kv.v[a.layer]);
-  attn_bf16x8 kr[CH], vr[CH];
-  auto fetch = [&](int kb) {
+  attn_bf16x8 kr[PF][CH], vr[PF][CH];
+  auto fetch = [&](int kb, attn_bf16x8 (&kx)[CH], attn_bf16x8 (&vx)[CH]) {
     const KVBlock blk = kv_block(a.kv, a.layer, b, g, kb);
     const bf16* kp = Kc + blk.k0 + sr * 64 + sc16;
     const bf16* vp = Vc + blk.v0 + (int64_t)sr * blk.vstride + sc16;
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
-      kr[c] = *reinterpret_cast<const attn_bf16x8*>(kp + 8 * c);
-      vr[c] = *reinterpret_cast<const attn_bf16x8*>(vp + 8 * c);
+      kx[c] = *reinterpret_cast<const attn_bf16x8*>(kp + 8 * c);
+      vx[c] = *reinterpret_cast<const attn_bf16x8*>(vp + 8 * c);
     }
   };
-  const int kb0 = tlo & ~63;
-  fetch(kb0);
-  for (int kb = kb0; kb <= thi; kb += 64) {
-    __syncthreads();  // the previous block's LDS reads are done
-    if (stager) {
+  auto block = [&](int kb, int buf, attn_bf16x8 (&kx)[CH], attn_bf16x8 (&vx)[CH]) {
 #pragma unroll
-      for (int c = 0; c < CH; ++c) {
-        *reinterpret_cast<attn_bf16x8*>(&Ks[sr][sc16 + 8 * c]) = kr[c];
-        // keys k0 .. k0 + 7 of the block: the two 4-key halves go to the slots of lanes
-        // kq and kq + 1 of the same key-tile parity
-        const int k0 = sc16 + 8 * c, w0 = k0 & 31, kqa = (w0 >> 2) & 3;
-        bf16* vrow = reinterpret_cast<bf16*>(&Vs[sr][(k0 & 32) + (w0 >> 4) * 4]);
-        *reinterpret_cast<attn_bf16x4*>(vrow + kqa * 8) =
-            __builtin_shufflevector(vr[c], vr[c], 0, 1, 2, 3);
-        *reinterpret_cast<attn_bf16x4*>(vrow + (kqa + 1) * 8) =
-            __builtin_shufflevector(vr[c], vr[c], 4, 5, 6, 7);
-      }
+    for (int c = 0; c < CH; ++c) {
+      *reinterpret_cast<attn_bf16x8*>(&Ks[buf][sr][sc16 + 8 * c]) = kx[c];
+      // keys k0 .. k0 + 7 of the block: the two 4-key halves go to the slots of lanes
+      // kq and kq + 1 of the same key-tile parity
+      const int k0 = sc16 + 8 * c, w0 = k0 & 31, kqa = (w0 >> 2) & 3;
+      bf16* vrow = reinterpret_cast<bf16*>(&Vs[buf][sr][(k0 & 32) + (w0 >> 4) * 4]);
+      *reinterpret_cast<attn_bf16x4*>(vrow + kqa * 8) =
+          __builtin_shufflevector(vx[c], vx[c], 0, 1, 2, 3);
+      *reinterpret_cast<attn_bf16x4*>(vrow + (kqa + 1) * 8) =
+          __builtin_shufflevector(vx[c], vx[c], 4, 5, 6, 7);
     }
-    __syncthreads();
-    if (kb + 64 <= thi) fetch(kb + 64);  // in flight during this block's products
+    // the other buffer's reads (the previous block's) are done once every wave is here
+    lds_barrier();
+    if (kb + 64 * PF <= thi) fetch(kb + 64 * PF, kx, vx);  // in flight during PF blocks' products
 
     attn_f32x4 sv[4][NQ];  // S^T tile (key tile kt, query tile nt)
 #pragma unroll
     for (int kt = 0; kt < 4; ++kt) {
-      const attn_bf16x8 k0 = *reinterpret_cast<const attn_bf16x8*>(&Ks[kt * 16 + m16][kq * 8]);
-      const attn_bf16x8 k1 = *reinterpret_cast<const attn_bf16x8*>(&Ks[kt * 16 + m16][32 + kq * 8]);
+      const attn_bf16x8 k0 = *reinterpret_cast<const attn_bf16x8*>(&Ks[buf][kt * 16 + m16][kq * 8]);
+      const attn_bf16x8 k1 = *reinterpret_cast<const attn_bf16x8*>(&Ks[buf][kt * 16 + m16][32 + kq * 8]);
 #pragma unroll
       for (int nt = 0; nt < NQ; ++nt) {
         attn_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
@@ -1447,38 +1445,46 @@ __global__ void __launch_bounds__(256 * (4 / NQ), 4) attn_prefill_mfma_kernel(At
         sv[kt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1, qb[nt][1], acc, 0, 0, 0);
       }
     }
-    const bool full = kb >= flo && kb + 63 <= fhi;  // uniform per block
+    if (!(kb >= flo && kb + 63 <= fhi)) {  // uniform per block
+#pragma unroll
+      for (int nt = 0; nt < NQ; ++nt)
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const int key = kb + kt * 16 + kq * 4 + j;
+            if (key < qlo[nt] || key > qhi[nt]) sv[kt][nt][j] = -INFINITY;
+          }
+    }
     attn_bf16x8 pb[NQ][2];
 #pragma unroll
     for (int nt = 0; nt < NQ; ++nt) {
+      // (score x scale) is rounded before the maximum is subtracted: not one fma
+#pragma clang fp contract(off)
       float mx = -INFINITY;
 #pragma unroll
       for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          float v = sv[kt][nt][j] * sl2;
-          if (!full) {
-            const int key = kb + kt * 16 + kq * 4 + j;
-            v = (key >= qlo[nt] && key <= qhi[nt]) ? v : -INFINITY;
-          }
-          sv[kt][nt][j] = v;
-          mx = fmaxf(mx, v);
-        }
+        for (int j = 0; j < 4; ++j) mx = fmaxf(mx, sv[kt][nt][j]);
       mx = fmaxf(mx, swz_xor16(mx));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-      const float mnew = fmaxf(mrun[nt], mx);
-      const float muse = mnew == -INFINITY ? 0.f : mnew;
-      const float f = __builtin_amdgcn_exp2f(mrun[nt] - muse);
-      mrun[nt] = mnew;
-      float ls = lrun[nt] * f;
+      mx = fmaxf(mx, __shfl_xor(mx, 32, 64)) * sl2;
+      // the output is scaled only where some query's maximum grew (by 1 everywhere else)
+      float f = 1.f;
+      if (__any(mx > mrun[nt])) {
+        const float mnew = fmaxf(mrun[nt], mx);
+        f = mnew == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(mrun[nt] - mnew);
+        mrun[nt] = mnew;
 #pragma unroll
-      for (int mt = 0; mt < 4; ++mt) o[mt][nt] *= f;
+        for (int mt = 0; mt < 4; ++mt) o[mt][nt] *= f;
+      }
+      const float muse = mrun[nt] == -INFINITY ? 0.f : mrun[nt];
+      float ls = 0.f;
 #pragma unroll
       for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          const float p = __builtin_amdgcn_exp2f(sv[kt][nt][j] - muse);
-          ls += p;
+          const float p = __builtin_amdgcn_exp2f(sv[kt][nt][j] * sl2 - muse);
+          ls = kt + j == 0 ? fmaf(lrun[nt], f, p) : ls + p;
           pb[nt][kt >> 1][(kt & 1) * 4 + j] = (__bf16)p;
         }
       lrun[nt] = ls;
@@ -1487,11 +1493,22 @@ __global__ void __launch_bounds__(256 * (4 / NQ), 4) attn_prefill_mfma_kernel(At
     for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks) {
-        const attn_bf16x8 av = *reinterpret_cast<const attn_bf16x8*>(&Vs[mt * 16 + m16][ks * 32 + kq * 8]);
+        const attn_bf16x8 av = *reinterpret_cast<const attn_bf16x8*>(&Vs[buf][mt * 16 + m16][ks * 32 + kq * 8]);
 #pragma unroll
         for (int nt = 0; nt < NQ; ++nt)
           o[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, pb[nt][ks], o[mt][nt], 0, 0, 0);
       }
+  };
+  const int kb0 = tlo & ~63;
+  fetch(kb0, kr[0], vr[0]);
+  if (PF > 1 && kb0 + 64 <= thi) fetch(kb0 + 64, kr[PF - 1], vr[PF - 1]);
+  if constexpr (PF > 1) {
+    for (int kb = kb0; kb <= thi; kb += 128) {
+      block(kb, 0, kr[0], vr[0]);
+      if (kb + 64 <= thi) block(kb + 64, 1, kr[1], vr[1]);
+    }
+  } else {
+    for (int kb = kb0, buf = 0; kb <= thi; kb += 64, buf ^= 1) block(kb, buf, kr[0], vr[0]);
   }
   // lane holds O[query q0 + 16 nt + m16][dims 16 mt + 4 kq + j]
 #pragma unroll
@@ -1665,50 +1682,64 @@ __global__ void __launch_bounds__(256) router_prefill_kernel(RouterArgs a) {
 // 128 rows (16 x 2048 tokens: 28.1 -> 21.4 us per launch against every wave loading and
 // converting them itself). The logits, rounded to bf16, go through LDS to the shared top-k
 // routine (one lane per row), so routing is the same as router_prefill_kernel's.
-constexpr int kRouterWaves = 8;     // 16-row tiles per workgroup
+// All 8 waves stage; waves 0 .. RW - 1 compute, so that a short prompt's rows spread over the
+// CUs. The rows' and the weights' loads all go out before the first is used (KS = D / 32).
+constexpr int kRouterWaves = 8;
 constexpr int kRouterMaxD = 1024;   // model widths the staged weights cover
+template <int KS, int RW>
 __global__ void __launch_bounds__(64 * kRouterWaves) router_prefill_mfma_kernel(RouterArgs a) {
   // the pulse's weights, rounded to bf16 once per workgroup, in B-operand order: k step t,
   // lane (expert m16, k chunk kq) -> W[m16][32 t + 8 kq .. + 7] (zero for m16 >= E)
-  __shared__ attn_bf16x8 sw[kRouterMaxD / 32][64];
-  __shared__ float lg[kRouterWaves][16][17];
+  __shared__ attn_bf16x8 sw[KS][64];
+  __shared__ float lg[RW][16][17];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int m16 = lane & 15, kq = lane >> 4;
-  const int r0 = ((int)blockIdx.x * kRouterWaves + wv) * 16;
-  const int D = a.D, E = a.E, KS = D / 32;
+  const int r0 = ((int)blockIdx.x * RW + wv) * 16;
+  constexpr int D = 32 * KS;
+  const int E = a.E;
+  const bool rows = RW == kRouterWaves || wv < RW;
+  const attn_bf16x8 zero = {};
+  // the first half of the rows' loads goes out ahead of the weight staging, the second after
+  constexpr int KH = KS / 2;
   const bf16* xp = reinterpret_cast<const bf16*>(a.x) +
                    (int64_t)min(r0 + m16, a.m_fixed - 1) * D + kq * 8;
-  const attn_bf16x8 zero = {};
-  // the first rows' loads go out ahead of the weight staging
-  attn_bf16x8 xa[8];
+  attn_bf16x8 xa[KS];
+  if (rows) {
 #pragma unroll
-  for (int u = 0; u < 8; ++u) xa[u] = *reinterpret_cast<const attn_bf16x8*>(xp + 32 * u);
+    for (int u = 0; u < KH; ++u) xa[u] = *reinterpret_cast<const attn_bf16x8*>(xp + 32 * u);
+  }
   const float* wbase = a.w + (int64_t)a.pulse * E * D;
-  for (int f = tid; f < KS * 64; f += 64 * kRouterWaves) {
-    const int t = f >> 6, l = f & 63, ex = l & 15;
+  constexpr int NF = KS * 64 / (64 * kRouterWaves);  // staged fragments per thread
+  float4 w0[NF], w1[NF];
+#pragma unroll
+  for (int i = 0; i < NF; ++i) {
+    const int f = tid + i * 64 * kRouterWaves, t = f >> 6, l = f & 63, ex = l & 15;
     const float* src = wbase + (int64_t)min(ex, E - 1) * D + t * 32 + (l >> 4) * 8;
-    const float4 w0 = *reinterpret_cast<const float4*>(src);
-    const float4 w1 = *reinterpret_cast<const float4*>(src + 4);
+    w0[i] = *reinterpret_cast<const float4*>(src);
+    w1[i] = *reinterpret_cast<const float4*>(src + 4);
+  }
+  if (rows) {
+#pragma unroll
+    for (int u = KH; u < KS; ++u) xa[u] = *reinterpret_cast<const attn_bf16x8*>(xp + 32 * u);
+  }
+#pragma unroll
+  for (int i = 0; i < NF; ++i) {
+    const int f = tid + i * 64 * kRouterWaves, l = f & 63;
     attn_bf16x8 v;
-    v[0] = (__bf16)w0.x; v[1] = (__bf16)w0.y; v[2] = (__bf16)w0.z; v[3] = (__bf16)w0.w;
-    v[4] = (__bf16)w1.x; v[5] = (__bf16)w1.y; v[6] = (__bf16)w1.z; v[7] = (__bf16)w1.w;
-    sw[t][l] = ex < E ? v : zero;
+    v[0] = (__bf16)w0[i].x; v[1] = (__bf16)w0[i].y; v[2] = (__bf16)w0[i].z; v[3] = (__bf16)w0[i].w;
+    v[4] = (__bf16)w1[i].x; v[5] = (__bf16)w1[i].y; v[6] = (__bf16)w1[i].z; v[7] = (__bf16)w1[i].w;
+    sw[f >> 6][l] = (l & 15) < E ? v : zero;
   }
-  __syncthreads();
+  lds_barrier();
+  if (!rows) return;
   attn_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  for (int k = 0; k < D; k += 256) {
-    if (k > 0) {
 #pragma unroll
-      for (int u = 0; u < 8; ++u) xa[u] = *reinterpret_cast<const attn_bf16x8*>(xp + k + 32 * u);
-    }
-#pragma unroll
-    for (int u = 0; u < 8; ++u)
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[u], sw[(k >> 5) + u][lane], acc, 0, 0, 0);
-  }
-  // lane holds the logits of rows 4 kq + j for expert m16
+  for (int u = 0; u < KS; ++u)
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[u], sw[u][lane], acc, 0, 0, 0);
+  // lane holds the logits of rows 4 kq + j for expert m16; the wave reads its own slice back
 #pragma unroll
   for (int j = 0; j < 4; ++j) lg[wv][kq * 4 + j][m16] = rnd<bf16>(acc[j]);
-  __syncthreads();
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   if (lane < 16 && r0 + lane < a.m_fixed)
     route_topk<bf16>(lg[wv][lane], E, a.K, a.bias + (int64_t)a.pulse * E, r0 + lane, a);
 }
@@ -1723,7 +1754,8 @@ __global__ void __launch_bounds__(64 * kRouterWaves) router_prefill_mfma_kernel(
 // LDS atomic per wave; prefill of 16 x 2048 tokens: 97 -> 84 us per launch). Under
 // capacity every one is kept; over capacity the C first in (key asc, flat index asc) order
 // are: the C-th smallest key found by bisection over the keys' ordered bits, in LDS when
-// staged, else over the sequence's assignments in memory, and the assignments on that key
+// staged (from [e - 0.5, e], which holds every key: 1 x 517 tokens 14.9 -> 12.8 us; ranking
+// each of up to 512 keys against all 23.8), else over the sequence's assignments in memory, and the assignments on that key
 // ranked by flat index. The block then reserves its kept count in the expert's list with
 // one atomic and writes its entries there.
 __device__ int block_excl_scan_int(int v, int* scratch, int* total) {
@@ -1831,7 +1863,8 @@ __global__ void __launch_bounds__(256) prefill_select_kernel(
     int below = 0;
     bool tie_bits = false, lone_tie = false;
     if (n > C) {
-      uint32_t lo = 0u, hi = 0xffffffffu;
+      // the keys lie in [e - 0.5, e]
+      uint32_t lo = ordered_bits((float)e - 0.5f), hi = ordered_bits((float)e);
       while (lo < hi) {
         const uint32_t mid = lo + ((hi - lo) >> 1);
         int c = 0;
@@ -2266,15 +2299,24 @@ int launch_attn_decode(const AttnArgs& a, int dtype, int max_rows, hipStream_t s
   PULSAR_LAUNCH_CHECK();
   return PULSAR_OK;
 }
+constexpr int64_t kPrefillBlocks = 256;
 int launch_attn_prefill(const AttnArgs& a, int dtype, int B, hipStream_t s) {
   const int ntile = (a.prefill_T + 63) / 64;
   if (a.H != 4 * a.Hkv)
     return fail(PULSAR_ERR_UNSUPPORTED, "prefill attention: four query heads per kv head");
   if (dtype == PULSAR_BF16) {
-    // two 16-query tiles per wave: each K and V fragment read from LDS feeds two products
-    // (16 x 2048 tokens: 289 -> 260 us per launch against one tile per wave at 16 waves;
-    // 352 us with two tiles at 136 registers, where one workgroup fills a CU)
-    attn_prefill_mfma_kernel<2><<<dim3(B * ntile, a.Hkv), 512, 0, s>>>(a);
+    // the largest query tile that leaves a workgroup for every CU (one tile of a short prompt
+    // is a chain over all its key blocks): each key and value fragment read from LDS feeds
+    // as many products as a wave has query tiles. Results do not depend on the tile. 1 x 517
+    // tokens: 22.3 us in 64-query tiles (36 workgroups), 10.6 in 16-query ones (132).
+    auto grid = [&](int q) { return dim3((unsigned)(B * ((a.prefill_T + q - 1) / q)), (unsigned)a.Hkv); };
+    auto blocks = [&](int q) { return (int64_t)grid(q).x * a.Hkv; };
+    if (blocks(64) >= kPrefillBlocks)
+      attn_prefill_mfma_kernel<2, 2><<<grid(64), 512, 0, s>>>(a);
+    else if (blocks(32) >= kPrefillBlocks)
+      attn_prefill_mfma_kernel<2, 1><<<grid(32), 256, 0, s>>>(a);
+    else
+      attn_prefill_mfma_kernel<1, 1><<<grid(16), 256, 0, s>>>(a);
     PULSAR_LAUNCH_CHECK();
     return PULSAR_OK;
   }
@@ -2310,10 +2352,24 @@ int launch_norm_router(const RouterArgs& a, int dtype, int max_rows, hipStream_t
 }
 int launch_router_prefill(const RouterArgs& a, int dtype, hipStream_t s) {
   if (a.E > 32) return fail(PULSAR_ERR_UNSUPPORTED, "router: at most 32 experts");
-  if (dtype == PULSAR_BF16 && a.E <= 16 && a.D % 256 == 0 && a.D <= kRouterMaxD) {
-    const int rows = 16 * kRouterWaves;
-    router_prefill_mfma_kernel<<<dim3((unsigned)((a.m_fixed + rows - 1) / rows)), 64 * kRouterWaves,
-                                 0, s>>>(a);
+  if (dtype == PULSAR_BF16 && a.E <= 16 && (a.D == 256 || a.D == 512 || a.D == 1024)) {
+    static_assert(kRouterMaxD == 1024, "the widths above");
+    if (a.m_fixed <= 0) return PULSAR_OK;
+    // 16-row tiles per workgroup: as many as leave a workgroup for every CU (517 rows: 16.5 us
+    // at 8 tiles, 5 workgroups; 11.2 at one)
+    const int tiles = (a.m_fixed + 15) / 16;
+    auto run = [&](auto ks) {
+      constexpr int KS = decltype(ks)::value;
+      if (tiles >= 8 * 256)
+        router_prefill_mfma_kernel<KS, 8><<<(unsigned)((tiles + 7) / 8), 64 * kRouterWaves, 0, s>>>(a);
+      else if (tiles >= 2 * 256)
+        router_prefill_mfma_kernel<KS, 4><<<(unsigned)((tiles + 3) / 4), 64 * kRouterWaves, 0, s>>>(a);
+      else
+        router_prefill_mfma_kernel<KS, 1><<<(unsigned)tiles, 64 * kRouterWaves, 0, s>>>(a);
+    };
+    if (a.D == 256) run(std::integral_constant<int, 8>{});
+    else if (a.D == 512) run(std::integral_constant<int, 16>{});
+    else run(std::integral_constant<int, 32>{});
     PULSAR_LAUNCH_CHECK();
     return PULSAR_OK;
   }

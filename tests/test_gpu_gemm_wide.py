@@ -1,7 +1,7 @@
-"""The prefill GEMMs' tile shapes: every shape sums an output's K in the same order, so a
-sequence's prefill logits are the same bits in batches small and large enough to take each of
-them (64 x 64 to 128 x 256 tiles), and a step's output head gives what the block's rows give
-alone."""
+"""The prefill kernels' tile shapes: every GEMM shape sums an output's K in the same order, and
+a query's attention and a row's routing do not depend on the tile or workgroup that holds
+them, so a sequence's prefill logits are the same bits in batches small and large enough to
+take each shape."""
 
 from __future__ import annotations
 
@@ -25,7 +25,7 @@ def model():
     return DeviceModel(cfg, W.synthetic_state(cfg, seed=3), torch.bfloat16)
 
 
-@pytest.mark.parametrize("T", [128, 131, 193])
+@pytest.mark.parametrize("T", [128, 131, 193, 260])
 def test_prefill_logits_do_not_depend_on_the_tile_shape(model, T):
     V = model.cfg.vocab_size
     prompts = np.stack([W.uniform_ids(b, "wide", T, V) for b in range(128)])
@@ -37,7 +37,8 @@ def test_prefill_logits_do_not_depend_on_the_tile_shape(model, T):
             return eng.logits(B)
 
     # tiles of the widest projection (1552 columns): 128 rows take 64 x 64 tiles, 2000 rows
-    # 64 x 128, 4000 rows 128 x 128, 16384 rows and more 128 x 256
+    # 64 x 128, 4000 rows 128 x 128, 16384 rows and more 128 x 256; attention in 16, 32 and 64
+    # queries; the router in 1, 4 and (260 tokens) 8 row tiles
     sets = {B: logits(B) for B in (1, 16, 32, 128)}
     for B, got in sets.items():
         assert np.isfinite(got).all()
