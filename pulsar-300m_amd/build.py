@@ -1,9 +1,10 @@
-"""Build libpulsar_hip.so (gfx950) from csrc/ with hipcc, in place.
+"""Build libpulsar_hip.so (gfx950) from csrc/ with hipcc, and the op surface's native half
+(_ops.so, host code against torch's headers), in place.
 
     python pulsar-300m_amd/build.py [--jobs N]
 
-Objects are compiled in parallel into _build/ next to this file; the shared library is
-written to pulsar_cuda/libpulsar_hip.so, where the pulsar_cuda package loads it.
+Objects are compiled in parallel into _build/ next to this file; the shared libraries are
+written to pulsar_cuda/, where the pulsar_cuda package loads them.
 """
 
 from __future__ import annotations
@@ -17,6 +18,7 @@ from concurrent.futures import ThreadPoolExecutor
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "pulsar_cuda", "libpulsar_hip.so")
+OPS_OUT = os.path.join(HERE, "pulsar_cuda", "_ops.so")
 BUILD = os.path.join(HERE, "_build")
 SOURCES = ["ops.hip", "gemm.hip", "gemm_wide.hip", "rows.hip", "sample.hip", "engine.hip", "backward.hip"]
 ARCH = os.environ.get("PULSAR_HIP_ARCH", "gfx950")
@@ -38,17 +40,51 @@ def _compile(src: str) -> str:
     return obj
 
 
-def build(jobs: int = 8) -> str:
-    os.makedirs(BUILD, exist_ok=True)
-    with ThreadPoolExecutor(max(1, jobs)) as ex:
-        objs = list(ex.map(_compile, SOURCES))
-    tmp = OUT + ".tmp"
-    cmd = [HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", tmp]
+def _run(cmd: list, what: str) -> None:
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         sys.stderr.write(r.stdout + r.stderr)
-        raise RuntimeError("link failed")
+        raise RuntimeError(f"{what} failed")
+
+
+def _compile_ops() -> str:
+    """Host code of the op surface, against the headers of the installed torch."""
+    import sysconfig
+
+    import torch
+
+    t = os.path.dirname(torch.__file__)
+    obj = os.path.join(BUILD, "ops_torch.o")
+    abi = int(torch._C._GLIBCXX_USE_CXX11_ABI)
+    _run([HIPCC, "-x", "c++", "-O2", "-std=c++17", "-fPIC", "-w", "-DUSE_ROCM=1",
+          "-D__HIP_PLATFORM_AMD__=1", f"-D_GLIBCXX_USE_CXX11_ABI={abi}", f"-I{t}/include",
+          f"-I{t}/include/torch/csrc/api/include", "-I" + sysconfig.get_path("include"),
+          "-I" + os.path.join(os.path.dirname(os.path.dirname(HIPCC)), "include"),
+          "-c", os.path.join(CSRC, "ops_torch.cpp"), "-o", obj], "ops_torch.cpp")
+    return obj
+
+
+def _link_ops(obj: str) -> None:
+    import torch
+
+    t = os.path.join(os.path.dirname(torch.__file__), "lib")
+    tmp = OPS_OUT + ".tmp"
+    _run([HIPCC, "-shared", "-fPIC", "-no-hip-rt", obj, "-o", tmp, f"-L{t}", "-lc10", "-lc10_hip",
+          "-ltorch_cpu", "-ltorch_python", "-L" + os.path.dirname(OUT), "-l:libpulsar_hip.so",
+          "-Wl,-rpath,$ORIGIN"], "link of _ops.so")
+    os.replace(tmp, OPS_OUT)
+
+
+def build(jobs: int = 8) -> str:
+    os.makedirs(BUILD, exist_ok=True)
+    with ThreadPoolExecutor(max(1, jobs)) as ex:
+        ops = ex.submit(_compile_ops)
+        objs = list(ex.map(_compile, SOURCES))
+        ops_obj = ops.result()
+    tmp = OUT + ".tmp"
+    _run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", tmp], "link")
     os.replace(tmp, OUT)
+    _link_ops(ops_obj)
     return OUT
 
 

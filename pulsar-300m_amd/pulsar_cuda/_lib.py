@@ -160,6 +160,18 @@ def load(path: str = LIB_PATH) -> ctypes.CDLL:
     return lib
 
 
+def load_ops():
+    """The op surface's native half (the extension module _ops), once the library is loaded."""
+    path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_ops.so")
+    if not os.path.exists(path):
+        raise RuntimeError(
+            f"_ops.so not found at {path}; build it with "
+            "`python pulsar-300m_amd/build.py` (or __graft_entry__.build())")
+    from . import _ops
+
+    return _ops
+
+
 def check(rc: int) -> None:
     if rc != PULSAR_OK:
         msg = load().pulsar_last_error().decode("utf-8", "replace")
