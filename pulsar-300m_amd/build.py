@@ -20,7 +20,7 @@ CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "pulsar_cuda", "libpulsar_hip.so")
 OPS_OUT = os.path.join(HERE, "pulsar_cuda", "_ops.so")
 BUILD = os.path.join(HERE, "_build")
-SOURCES = ["ops.hip", "gemm.hip", "gemm_wide.hip", "rows.hip", "sample.hip", "engine.hip", "backward.hip"]
+SOURCES = ["ops.hip", "gemm.hip", "gemm_wide.hip", "gemm_f32.hip", "rows.hip", "sample.hip", "engine.hip", "backward.hip"]
 ARCH = os.environ.get("PULSAR_HIP_ARCH", "gfx950")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [

@@ -133,9 +133,14 @@ struct GemmArgs {
 
 int launch_gemm(const GemmArgs& a, int dtype, int epi, int groups, int max_rows,
                 hipStream_t s);
+// fp32 (what launch_gemm and launch_gemm_wide call for it): tiles on the matrix cores for the
+// rows of a prompt, or a wave per column. The two sum K in different orders.
+int launch_gemm_f32(const GemmArgs& a, int epi, int groups, int max_rows, bool tiles,
+                    hipStream_t s);
 // Same contract, for row sets of hundreds to tens of thousands of rows (prefill): bf16
 // launches without a fused all-rows group use output tiles of 64 x 64 to 128 x 256, with
-// results that do not depend on the tile; others fall back to launch_gemm. The two kernels
+// results that do not depend on the tile; others fall back to launch_gemm (fp32: 32 x 32
+// tiles). The kernels
 // sum K in different orders, so a caller that wants results independent of batch composition
 // picks one by a per-sequence property (prompt length).
 int launch_gemm_wide(const GemmArgs& a, int dtype, int epi, int groups, int max_rows,

@@ -30,7 +30,7 @@ struct Engine {
   RowDesc* rows = nullptr;
   RowDesc* last_rows = nullptr;
   AttnUnit* units = nullptr;
-  int32_t* split_done = nullptr;  // [B][Hkv] decode attention split counters
+  int32_t* split_done = nullptr;  // [rows][Hkv] decode attention split counters (bf16: per unit)
   SeqState* state = nullptr;
   int32_t *lrow_seq = nullptr, *lrow_extra = nullptr, *argmax = nullptr, *draw = nullptr;
   uint32_t* lrow_ctr = nullptr;  // draft-block mode: per logits row draw counter
@@ -295,8 +295,8 @@ int create(const PulsarModelDesc& m, const PulsarEngineConfig& c, Engine** out) 
   PULSAR_TRY(x.alloc(&x.v_rows, sizeof(RowDesc) * x.P * MR));
   PULSAR_TRY(x.alloc(&x.v_ctl, sizeof(StepCtl) * x.P));
   PULSAR_TRY(x.alloc(&x.v_units, sizeof(AttnUnit) * x.P * x.B));
-  PULSAR_TRY(x.alloc(&x.split_done, 4 * (size_t)x.B * x.Hkv));
-  PULSAR_CHECK_HIP(hipMemset(x.split_done, 0, 4 * (size_t)x.B * x.Hkv));
+  PULSAR_TRY(x.alloc(&x.split_done, 4 * (size_t)MR * x.Hkv));
+  PULSAR_CHECK_HIP(hipMemset(x.split_done, 0, 4 * (size_t)MR * x.Hkv));
   PULSAR_TRY(x.alloc(&x.state, sizeof(SeqState) * x.B));
   PULSAR_TRY(x.alloc(&x.lrow_seq, 4 * MR));
   PULSAR_TRY(x.alloc(&x.lrow_extra, 4 * MR * kMaxExtra));
@@ -681,8 +681,8 @@ int enqueue_pass(Engine& e, const StepCtl* ctl, const RowDesc* rows, const AttnU
     ca.next_norm = l + 1 < e.L ? m.attn_norm[l + 1] : nullptr;
     ca.xn = e.xn;
     ca.eps = m.rms_eps;
-    if (fuse_post && l + 1 == e.L) {
-      // bf16: the last layer's combine also does the pulse output (no separate launch)
+    if (l + 1 == e.L) {
+      // the last layer's combine also does the pulse output (no separate launch)
       ca.h_in = e.h_in;
       ca.res_scale = m.res_scale;
       ca.hout_state = e.hout_state;
@@ -691,21 +691,6 @@ int enqueue_pass(Engine& e, const StepCtl* ctl, const RowDesc* rows, const AttnU
       ca.xn_final = e.xn_final;
     }
     PULSAR_TIMED(PC_COMBINE, launch_moe_combine(ca, dt, MR, s));
-  }
-  if (!fuse_post) {
-    PulseOutputArgs po{};
-    po.ctl = ctl;
-    po.rows = rows;
-    po.D = D;
-    po.slots = e.S;
-    po.eps = m.rms_eps;
-    po.h_in = e.h_in;
-    po.h = e.h;
-    po.res_scale = m.res_scale;
-    po.hout_state = e.hout_state;
-    po.final_norm = m.final_norm;
-    po.xn_final = e.xn_final;
-    PULSAR_TIMED(PC_OUTPUT, launch_pulse_output(po, dt, MR, s));
   }
   if (!head) return PULSAR_OK;
   GemmArgs g = gemm_base(e);
@@ -941,6 +926,8 @@ int first_token(Engine& e, uint64_t seed, hipStream_t s) {
 }
 
 constexpr int kWidePromptLen = 128;
+// fp32: prompts of this many tokens or more run the GEMMs in 32-row tiles on the matrix cores
+constexpr int kWidePromptLenF32 = 16;
 
 int prefill(Engine& e, const int32_t* host_ids, int Bq, int T, hipStream_t s) {
   const PulsarModelDesc& m = e.m;
@@ -987,7 +974,7 @@ int prefill(Engine& e, const int32_t* host_ids, int Bq, int T, hipStream_t s) {
   const int64_t lstride = (int64_t)e.R * e.K;
   // Wide-tile GEMMs for prompts of kWidePromptLen tokens or more. The choice depends on the
   // prompt length only, so a sequence gets the same arithmetic alone or in a batch.
-  const bool wide = T >= kWidePromptLen;
+  const bool wide = T >= (dt == PULSAR_BF16 ? kWidePromptLen : kWidePromptLenF32);
   auto gemm_rows = [&](const GemmArgs& g, int epi, int groups, int rows) {
     return wide ? launch_gemm_wide(g, dt, epi, groups, rows, s)
                 : launch_gemm(g, dt, epi, groups, rows, s);

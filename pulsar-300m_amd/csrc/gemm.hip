@@ -11,7 +11,7 @@
 //
 // Prefill and other wide row sets: gemm_wide.hip.
 //
-// fp32: one wave per output column, lanes split K with 128-bit loads, wave64 reduction.
+// fp32: gemm_f32.hip.
 #include <algorithm>
 
 #include "gemm_common.h"
@@ -27,65 +27,6 @@ __device__ __forceinline__ bf16x8_t load_bf16x8(const bf16* p) {
 // out of the caches what later kernels read again (attention keys/values, activations).
 __device__ __forceinline__ bf16x8_t load_bf16x8_nt(const bf16* p) {
   return __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(p));
-}
-
-// Resolve the (A row, C row) pairs of this workgroup's 32-row tile into LDS.
-// Returns the number of valid rows (0 => nothing to do).
-__device__ int resolve_rows(const GemmArgs& g, int group, int tile, int* a_row, int* c_row) {
-  __shared__ int s_n;
-  const int mode = (g.has_g0 && group < 0) ? ROWS_ALL : g.row_mode;
-  if (threadIdx.x == 0) {
-    int n = 0;
-    switch (mode) {
-      case ROWS_PULSE: {
-        const int cnt = g.ctl->pulse_count[group];
-        n = cnt - tile * 32;
-        break;
-      }
-      case ROWS_LIST:
-        n = g.list_count[group] - tile * 32;
-        break;
-      case ROWS_ALL: {
-        const int tot = g.ctl ? g.ctl->n_rows : g.m_fixed;
-        n = tot - tile * 32;
-        break;
-      }
-      case ROWS_LOGITS:
-        n = g.ctl->n_lrows - tile * 32;
-        break;
-    }
-    s_n = n < 0 ? 0 : (n > 32 ? 32 : n);
-  }
-  __syncthreads();
-  const int n = s_n;
-  if (threadIdx.x < 32) {
-    const int m = threadIdx.x;
-    int ar = -1, cr = -1;
-    if (m < n) {
-      const int i = tile * 32 + m;
-      switch (mode) {
-        case ROWS_PULSE:
-          ar = cr = g.ctl->pulse_start[group] + i;
-          break;
-        case ROWS_LIST: {
-          const int e = g.list[(int64_t)group * g.list_stride + i];
-          ar = e / g.a_div;
-          cr = e;
-          break;
-        }
-        case ROWS_ALL:
-          ar = cr = i;
-          break;
-        case ROWS_LOGITS:
-          ar = cr = i;
-          break;
-      }
-    }
-    a_row[m] = ar;
-    c_row[m] = cr < 0 ? -1 : cr + g.c_row_offset;
-  }
-  __syncthreads();
-  return n;
 }
 
 // Workgroup: 16 output columns of one group; 8 waves split K (few registers per wave, so
@@ -409,46 +350,6 @@ __global__ void __launch_bounds__(64 * kGemmWaves) gemm_bf16_kernel(GemmArgs g) 
 #undef PULSAR_LOAD_W_REST
 }
 
-// fp32: 4 waves per workgroup, one output column per wave, 32-row tile.
-template <int EPI>
-__global__ void __launch_bounds__(256) gemm_f32_kernel(GemmArgs g) {
-  constexpr bool kPair = (EPI == EPI_SWIGLU);
-  __shared__ int a_row[32], c_row[32];
-  const int group = (int)blockIdx.y + g.group_offset - (g.has_g0 ? 1 : 0);
-  const bool g0 = group < 0;
-  const int N = g0 ? g.N0 : g.N;
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int col = blockIdx.x * 4 + wv;
-  if (blockIdx.x * 4 >= N) return;
-  const int n = resolve_rows(g, group, blockIdx.z, a_row, c_row);
-  if (n == 0 || col >= N) return;
-  const float* A = reinterpret_cast<const float*>(g0 ? g.A0 : g.A);
-  const int64_t lda = g0 ? g.lda0 : g.lda, ldw = g0 ? g.ldw0 : g.ldw;
-  const float* W = g0 ? reinterpret_cast<const float*>(g.W0)
-                      : reinterpret_cast<const float*>(g.W) + (int64_t)group * g.w_group_stride;
-  void* Cout = g0 ? g.C0 : g.C;
-  const int64_t ldc = g0 ? g.ldc0 : g.ldc;
-  const float* w0 = W + (int64_t)col * ldw;
-  const float* w1 = W + (int64_t)(N + col) * ldw;
-  const int Kg = g0 ? g.K0 : g.K;
-  for (int r = 0; r < n; ++r) {
-    const float* a = A + (int64_t)a_row[r] * lda;
-    float s0 = 0.f, s1 = 0.f;
-    for (int k = lane * 4; k < Kg; k += 256) {
-      const float4 av = *reinterpret_cast<const float4*>(a + k);
-      const float4 bv = *reinterpret_cast<const float4*>(w0 + k);
-      s0 += av.x * bv.x + av.y * bv.y + av.z * bv.z + av.w * bv.w;
-      if constexpr (kPair) {
-        const float4 uv = *reinterpret_cast<const float4*>(w1 + k);
-        s1 += av.x * uv.x + av.y * uv.y + av.z * uv.z + av.w * uv.w;
-      }
-    }
-    s0 = wave_sum(s0);
-    if constexpr (kPair) s1 = wave_sum(s1);
-    if (lane == (r & 63)) epilogue<float>(g, EPI, group, Cout, ldc, c_row[r], col, s0, s1);
-  }
-}
-
 // Mid-size row sets (tens to a few hundred rows per group: block verifies, large decode
 // batches). A workgroup of 4 waves owns R = 64 RB rows of one group and CT weight column
 // tiles of 16 (CT = 4: 64 output columns, SwiGLU 32 gate columns and their 32 up twins;
@@ -693,55 +594,50 @@ constexpr int kTilesPerWorkgroup = 4;
 constexpr int kG0Split = 4;
 
 template <int EPI>
-int launch_one(const GemmArgs& a, int dtype, int groups, int max_rows, hipStream_t s) {
+int launch_one(const GemmArgs& a, int groups, int max_rows, hipStream_t s) {
   const int tiles = (max_rows + 31) / 32;
   if (tiles <= 0 || groups <= 0) return PULSAR_OK;
   int gy = groups + (a.has_g0 ? 1 : 0);
   const int nmax = a.has_g0 ? std::max(a.N, a.N0) : a.N;
   const int k0 = a.has_g0 ? a.K0 : a.K;
-  if (dtype == PULSAR_BF16) {
-    if (a.K != 256 && a.K != 512 && a.K != 1024 && a.K != 2048)
-      return fail(PULSAR_ERR_UNSUPPORTED, "gemm: K must be 256, 512, 1024 or 2048");
-    if (a.has_g0 && (a.row_mode != ROWS_LIST || a.ctl == nullptr))
-      return fail(PULSAR_ERR_INVALID,
-                  "gemm: the all-rows group fuses into list launches with a control block only");
-    if (k0 != a.K && k0 != 2 * a.K)
-      return fail(PULSAR_ERR_UNSUPPORTED, "gemm: the all-rows group needs K0 = K or 2K");
-    const int per_wg = a.row_mode == ROWS_PULSE ? 1 : kTilesPerWorkgroup;
-    const int gz = (tiles + per_wg - 1) / per_wg;
-    // the all-rows group: one row tile per workgroup, up to kG0Split rows of the grid
-    const int s0 = a.has_g0 ? std::min(kG0Split, (tiles + gz - 1) / gz) : 0;
-    gy = groups + s0;
-    dim3 grid((unsigned)((nmax + 15) / 16), (unsigned)gy, (unsigned)gz);
-    GemmArgs ga = a;
-    ga.g0_split = s0;
-    ga.grid_x = (int)grid.x;
-    ga.grid_y = (int)grid.y;
-    ga.grid_z = (int)grid.z;
-    switch (a.row_mode) {
-      case ROWS_PULSE: launch_bf16_k<EPI, ROWS_PULSE, 1>(ga, grid, s); break;
-      case ROWS_LIST:
-        if (a.eager_w) {
-          if (EPI != EPI_SWIGLU || k0 != a.K)
-            return fail(PULSAR_ERR_UNSUPPORTED,
-                        "gemm: eager expert launches are SwiGLU with K0 == K");
-          if (a.a_rows < 1 || (a.has_g0 && a.a_rows0 < 1))
-            return fail(PULSAR_ERR_INVALID, "gemm: eager expert launches need A row counts");
-          if constexpr (EPI == EPI_SWIGLU) launch_bf16_k<EPI, ROWS_LIST, 1, true>(ga, grid, s);
-        } else {
-          if (k0 == a.K)
-            launch_bf16_k<EPI, ROWS_LIST, 1>(ga, grid, s);
-          else
-            launch_bf16_k<EPI, ROWS_LIST, 2>(ga, grid, s);
-        }
-        break;
-      case ROWS_ALL: launch_bf16_k<EPI, ROWS_ALL, 1>(ga, grid, s); break;
-      case ROWS_LOGITS: launch_bf16_k<EPI, ROWS_LOGITS, 1>(ga, grid, s); break;
-      default: return fail(PULSAR_ERR_INVALID, "gemm: row mode");
-    }
-  } else {
-    dim3 grid((unsigned)((nmax + 3) / 4), (unsigned)gy, (unsigned)tiles);
-    gemm_f32_kernel<EPI><<<grid, 256, 0, s>>>(a);
+  if (a.K != 256 && a.K != 512 && a.K != 1024 && a.K != 2048)
+    return fail(PULSAR_ERR_UNSUPPORTED, "gemm: K must be 256, 512, 1024 or 2048");
+  if (a.has_g0 && (a.row_mode != ROWS_LIST || a.ctl == nullptr))
+    return fail(PULSAR_ERR_INVALID,
+                "gemm: the all-rows group fuses into list launches with a control block only");
+  if (k0 != a.K && k0 != 2 * a.K)
+    return fail(PULSAR_ERR_UNSUPPORTED, "gemm: the all-rows group needs K0 = K or 2K");
+  const int per_wg = a.row_mode == ROWS_PULSE ? 1 : kTilesPerWorkgroup;
+  const int gz = (tiles + per_wg - 1) / per_wg;
+  // the all-rows group: one row tile per workgroup, up to kG0Split rows of the grid
+  const int s0 = a.has_g0 ? std::min(kG0Split, (tiles + gz - 1) / gz) : 0;
+  gy = groups + s0;
+  dim3 grid((unsigned)((nmax + 15) / 16), (unsigned)gy, (unsigned)gz);
+  GemmArgs ga = a;
+  ga.g0_split = s0;
+  ga.grid_x = (int)grid.x;
+  ga.grid_y = (int)grid.y;
+  ga.grid_z = (int)grid.z;
+  switch (a.row_mode) {
+    case ROWS_PULSE: launch_bf16_k<EPI, ROWS_PULSE, 1>(ga, grid, s); break;
+    case ROWS_LIST:
+      if (a.eager_w) {
+        if (EPI != EPI_SWIGLU || k0 != a.K)
+          return fail(PULSAR_ERR_UNSUPPORTED,
+                      "gemm: eager expert launches are SwiGLU with K0 == K");
+        if (a.a_rows < 1 || (a.has_g0 && a.a_rows0 < 1))
+          return fail(PULSAR_ERR_INVALID, "gemm: eager expert launches need A row counts");
+        if constexpr (EPI == EPI_SWIGLU) launch_bf16_k<EPI, ROWS_LIST, 1, true>(ga, grid, s);
+      } else {
+        if (k0 == a.K)
+          launch_bf16_k<EPI, ROWS_LIST, 1>(ga, grid, s);
+        else
+          launch_bf16_k<EPI, ROWS_LIST, 2>(ga, grid, s);
+      }
+      break;
+    case ROWS_ALL: launch_bf16_k<EPI, ROWS_ALL, 1>(ga, grid, s); break;
+    case ROWS_LOGITS: launch_bf16_k<EPI, ROWS_LOGITS, 1>(ga, grid, s); break;
+    default: return fail(PULSAR_ERR_INVALID, "gemm: row mode");
   }
   PULSAR_LAUNCH_CHECK();
   return PULSAR_OK;
@@ -823,22 +719,21 @@ int launch_gemm_mid(const GemmArgs& a, int dtype, int epi, int groups, int max_r
 int launch_gemm(const GemmArgs& a, int dtype, int epi, int groups, int max_rows, hipStream_t s) {
   if (a.K % 256 != 0)
     return fail(PULSAR_ERR_UNSUPPORTED, "gemm: K must be a multiple of 256");
+  if (dtype != PULSAR_BF16) return launch_gemm_f32(a, epi, groups, max_rows, false, s);
   switch (epi) {
-    case EPI_STORE: return launch_one<EPI_STORE>(a, dtype, groups, max_rows, s);
-    case EPI_QKVG: return launch_one<EPI_QKVG>(a, dtype, groups, max_rows, s);
-    case EPI_RESID: return launch_one<EPI_RESID>(a, dtype, groups, max_rows, s);
-    case EPI_SWIGLU: return launch_one<EPI_SWIGLU>(a, dtype, groups, max_rows, s);
-    case EPI_LOGITS:
-      if (dtype == PULSAR_BF16) {
-        // column pairs (c, N/2 + c) per workgroup
-        if (a.N % 32 != 0) return fail(PULSAR_ERR_UNSUPPORTED, "gemm: logits N % 32 != 0");
-        GemmArgs h = a;
-        h.N = a.N / 2;
-        return launch_one<EPI_LOGITS>(h, dtype, groups, max_rows, s);
-      }
-      return launch_one<EPI_LOGITS>(a, dtype, groups, max_rows, s);
-    case EPI_LOGITS_RAW: return launch_one<EPI_LOGITS_RAW>(a, dtype, groups, max_rows, s);
-    case EPI_SCALE: return launch_one<EPI_SCALE>(a, dtype, groups, max_rows, s);
+    case EPI_STORE: return launch_one<EPI_STORE>(a, groups, max_rows, s);
+    case EPI_QKVG: return launch_one<EPI_QKVG>(a, groups, max_rows, s);
+    case EPI_RESID: return launch_one<EPI_RESID>(a, groups, max_rows, s);
+    case EPI_SWIGLU: return launch_one<EPI_SWIGLU>(a, groups, max_rows, s);
+    case EPI_LOGITS: {
+      // column pairs (c, N/2 + c) per workgroup
+      if (a.N % 32 != 0) return fail(PULSAR_ERR_UNSUPPORTED, "gemm: logits N % 32 != 0");
+      GemmArgs h = a;
+      h.N = a.N / 2;
+      return launch_one<EPI_LOGITS>(h, groups, max_rows, s);
+    }
+    case EPI_LOGITS_RAW: return launch_one<EPI_LOGITS_RAW>(a, groups, max_rows, s);
+    case EPI_SCALE: return launch_one<EPI_SCALE>(a, groups, max_rows, s);
   }
   return fail(PULSAR_ERR_INVALID, "gemm: unknown epilogue");
 }

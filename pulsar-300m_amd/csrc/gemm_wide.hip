@@ -311,8 +311,8 @@ int launch_wide(const GemmArgs& a, int groups, int max_rows, hipStream_t s) {
 
 int launch_gemm_wide(const GemmArgs& a, int dtype, int epi, int groups, int max_rows,
                      hipStream_t s) {
-  if (dtype != PULSAR_BF16 || a.has_g0)
-    return launch_gemm(a, dtype, epi, groups, max_rows, s);
+  if (a.has_g0) return launch_gemm(a, dtype, epi, groups, max_rows, s);
+  if (dtype != PULSAR_BF16) return launch_gemm_f32(a, epi, groups, max_rows, true, s);
   if (groups <= 0) return PULSAR_OK;
   if (a.K % 256 != 0 || a.N % 16 != 0 || (epi == EPI_SWIGLU && a.N % 128 != 0))
     return fail(PULSAR_ERR_UNSUPPORTED, "gemm: wide tiles need K % 256 == 0 and N % 16 == 0 "

@@ -209,21 +209,31 @@ __global__ void __launch_bounds__(64) pulse_input_kernel(PulseInputArgs a) {
     float rv[EPL];
 #pragma unroll
     for (int c = 0; c < EPL; ++c) rv[c] = rnd<T>(hpv[c] * inv * sn[c]);
+    // 4 ranks' weights in flight at a time (one rank at a time: 19.6 us for 2 fp32
+    // rows of 1024; 8.7 so)
     float gh[RT];
+    constexpr int RB = EPL <= 16 ? 4 : 1;
 #pragma unroll
-    for (int j = 0; j < RT; ++j) {
-      const int jj = j < R ? j : 0;  // ranks past R load rank 0 and are dropped
-      float we[EPL], wr[EPL];
-      ldv<EPL>(wd + (int64_t)jj * 2 * D + i0, we);
-      ldv<EPL>(wd + (int64_t)jj * 2 * D + D + i0, wr);
-      float pe = 0.f, pr = 0.f;
+    for (int j0 = 0; j0 < RT; j0 += RB) {
+      float we[RB][EPL], wr[RB][EPL];
 #pragma unroll
-      for (int c = 0; c < EPL; ++c) {
-        pe += ev[c] * we[c];
-        pr += rv[c] * wr[c];
+      for (int j = 0; j < RB; ++j) {
+        const int jj = j0 + j < R ? j0 + j : 0;  // ranks past R load rank 0 and are dropped
+        ldv<EPL>(wd + (int64_t)jj * 2 * D + i0, we[j]);
+        ldv<EPL>(wd + (int64_t)jj * 2 * D + D + i0, wr[j]);
       }
-      gh[j] = 0.f;
-      if (EXACT || j < R) gh[j] = rnd<T>(rnd<T>(wave_sum(pe)) + rnd<T>(wave_sum(pr)));
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < RB; ++j) {
+        float pe = 0.f, pr = 0.f;
+#pragma unroll
+        for (int c = 0; c < EPL; ++c) {
+          pe += ev[c] * we[j][c];
+          pr += rv[c] * wr[j][c];
+        }
+        gh[j0 + j] = 0.f;
+        if (EXACT || j0 + j < R) gh[j0 + j] = rnd<T>(rnd<T>(wave_sum(pe)) + rnd<T>(wave_sum(pr)));
+      }
     }
 #pragma unroll
     for (int c = 0; c < EPL; ++c) {
@@ -478,116 +488,107 @@ __global__ void __launch_bounds__(256) qk_post_kernel(QKPostArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// Decode attention for fp32 caches (the bf16 path runs on the matrix cores below), split
-// over keys: block (row, kv head, split) serves the 4 query heads of the group over up to
-// 256 keys, 64 per wave. Lane l owns key group (l >> 3), i.e. keys
-// kbeg + (l >> 3) + 8i for i < 8, and dims 8*(l & 7) .. +8, so each K and V load is 128
-// contiguous bits and every 8 lanes read one 128-byte key row: the wave reads 1 KB of
-// contiguous cache per load instruction (V, stored dimension-major, is gathered per
-// element: this path is for exactness, not speed). Scores are reduced over the 8 lanes of a key
-// group, softmax statistics over the wave; partials (max, sum, acc[64]) per query head go
-// to `part` and the combine kernel merges the splits.
+// Row-wise attention over fp32 caches (the bf16 path runs on the matrix cores below): decode,
+// and prefill of prompts whose keys fit one block. Block (row, kv head, split) serves the 4
+// query heads of the group over up to 256 keys from a multiple of 64, one 64-key cache block
+// per wave (contiguous in both caches). Scores: lane l owns keys (l >> 3) + 8 i and dims
+// 8 (l & 7) .. + 7, so K loads are 16 bytes per lane and 1 KB contiguous per wave; the 8
+// lanes of a key sum by DPP and each then exponentiates one of the group's 8 keys. Output:
+// lane = dim, its 64 values of the dimension-major V block in 16 16-byte loads (gathered
+// element by element they took half the kernel's time), the probabilities broadcast from LDS.
+// All loads go out before the first use. Several splits: (max, sum, acc[64]) per head go to
+// `part` and the last block to count in merges them in split order, as in the bf16 kernel
+// (2 rows at 128-190 positions: 17.3 us and a combine launch of 4.6 -> 9.4 us).
 // ---------------------------------------------------------------------------
-template <typename T>
-__device__ __forceinline__ void load8v(const T* p, float* o, bool valid) {
-  if (valid) {
-    load8(p, o);
-  } else {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) o[i] = 0.f;
-  }
-}
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float v) { return v + dpp_mov<CTRL>(v); }
 
-template <typename T>
-__global__ void __launch_bounds__(256) attn_decode_kernel(AttnArgs a) {
+__global__ void __launch_bounds__(256) attn_rows_f32_kernel(AttnArgs a) {
   __shared__ float wm[4][4], wl[4][4];
   __shared__ float wacc[4][4][64];
-  const int r = blockIdx.x;
-  if (r >= a.ctl->n_rows) return;
-  const int g = blockIdx.y, s = blockIdx.z;
+  __shared__ __attribute__((aligned(16))) float pr[4][4][64];  // [wave][head][key]
+  __shared__ int s_last;
+  const int r = blockIdx.x, g = blockIdx.y, s = blockIdx.z;
   const RowDesc rd = a.rows[r];
+  if (r >= a.ctl->n_rows) return;
   const int pos = rd.pos;
-  const int lo = a.is_local ? max(0, pos - a.window + 1) : 0;
-  const int nkeys = pos - lo + 1;
-  const int nsplit = (nkeys + kSplitLen - 1) / kSplitLen;
+  int lo = a.is_local ? max(0, pos - a.window + 1) : 0, hi = pos;
+  if (a.prefill_T > 0) {
+    // the reference's top-left aligned causal mask over the last `window` keys of a prompt
+    // longer than the window
+    const bool quirk = a.is_local && a.prefill_T > a.window;
+    lo = quirk ? a.prefill_T - a.window : 0;
+    hi = quirk ? lo + min(pos, a.window - 1) : pos;
+  }
+  const int base = lo & ~63;
+  const int nsplit = (hi - base) / kSplitLen + 1;
   if (s >= nsplit) return;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int kg = lane >> 3, dc = lane & 7;
-  // q of the 4 heads, this lane's 8 dims
-  const T* q = reinterpret_cast<const T*>(a.qkv) + (int64_t)r * a.ldq + (g * 4) * 64 + dc * 8;
-  float qv[4][8];
-#pragma unroll
-  for (int h = 0; h < 4; ++h) load8(q + h * 64, qv[h]);
-  const int kbeg = lo + s * kSplitLen + wv * 64;
-  const T* Kc = reinterpret_cast<const T*>(a.kv.k[a.layer]);
-  const T* Vc = reinterpret_cast<const T*>(a.kv.v[a.layer]);
-  float kf[8][8], vf[8][8];
-  bool valid[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int key = kbeg + kg + 8 * i;
-    valid[i] = key <= pos;
-    const int64_t off = valid[i] ? kv_offset(a.kv, a.layer, rd.seq, g, key) + dc * 8 : 0;
-    load8v(Kc + off, kf[i], valid[i]);
-#pragma unroll
-    for (int d = 0; d < 8; ++d)
-      vf[i][d] = valid[i] ? ld(Vc, kv_offset_v(a.kv, a.layer, rd.seq, g, key, dc * 8 + d)) : 0.f;
-  }
-  float sc[4][8];
+  const int kb = base + s * kSplitLen + wv * 64;  // this wave's 64 keys
+  const bool live = kb <= hi;                     // uniform per wave
+  float m[4], l[4], o[4];
 #pragma unroll
   for (int h = 0; h < 4; ++h) {
+    m[h] = -INFINITY;
+    l[h] = o[h] = 0.f;
+  }
+  if (live) {
+    const float* q = reinterpret_cast<const float*>(a.qkv) + (int64_t)r * a.ldq + (g * 4) * 64 + dc * 8;
+    const KVBlock blk = kv_block(a.kv, a.layer, rd.seq, g, kb);
+    const float* Kp = reinterpret_cast<const float*>(a.kv.k[a.layer]) + blk.k0 + kg * 64 + dc * 8;
+    const float* Vp = reinterpret_cast<const float*>(a.kv.v[a.layer]) + blk.v0 + (int64_t)lane * blk.vstride;
+    float qv[4][8], kf[8][8], vf[64];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int h = 0; h < 4; ++h) ldv<8>(q + h * 64, qv[h]);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ldv<8>(Kp + i * 512, kf[i]);
+    ldv<64>(Vp, vf);
+    const int mine = kb + kg + 8 * dc;  // the key this lane exponentiates
+    const bool ok = mine >= lo && mine <= hi;
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+      float x = -INFINITY;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        float acc = 0.f;
+#pragma unroll
+        for (int d = 0; d < 8; ++d) acc += qv[h][d] * kf[i][d];
+        acc = dpp_add<0xB1>(acc);   // lane ^ 1
+        acc = dpp_add<0x4E>(acc);   // lane ^ 2
+        acc = dpp_add<0x141>(acc);  // mirror of 8 lanes: the other four's sum
+        if (dc == i) x = acc * a.scale;
+      }
+      if (!ok) x = -INFINITY;
+      const float mx = wave_max(x);
+      const float p = ok ? expf(x - mx) : 0.f;
+      m[h] = mx;
+      l[h] = wave_sum(p);
+      pr[wv][h][kg + 8 * dc] = p;
+    }
+    // the wave reads its own slice back
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (kb < lo || kb + 63 > hi) {  // keys outside the range: whatever the cache holds there
+#pragma unroll
+      for (int k = 0; k < 64; ++k)
+        if (kb + k < lo || kb + k > hi) vf[k] = 0.f;
+    }
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
       float acc = 0.f;
 #pragma unroll
-      for (int d = 0; d < 8; ++d) acc += qv[h][d] * kf[i][d];
-      // sum the 8 dim chunks of this key
-      acc += __shfl_xor(acc, 1, 64);
-      acc += __shfl_xor(acc, 2, 64);
-      acc += __shfl_xor(acc, 4, 64);
-      sc[h][i] = valid[i] ? acc * a.scale : -INFINITY;
+      for (int k = 0; k < 64; k += 4) {
+        const float4 p = *reinterpret_cast<const float4*>(&pr[wv][h][k]);
+        acc += p.x * vf[k];
+        acc += p.y * vf[k + 1];
+        acc += p.z * vf[k + 2];
+        acc += p.w * vf[k + 3];
+      }
+      o[h] = acc;
     }
   }
-  float m[4], l[4], o[4][8];
 #pragma unroll
-  for (int h = 0; h < 4; ++h) {
-    float mx = -INFINITY;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) mx = fmaxf(mx, sc[h][i]);
-    mx = fmaxf(mx, __shfl_xor(mx, 8, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    m[h] = mx;
-    float ls = 0.f;
-#pragma unroll
-    for (int d = 0; d < 8; ++d) o[h][d] = 0.f;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float p = valid[i] ? expf(sc[h][i] - mx) : 0.f;
-      ls += p;
-#pragma unroll
-      for (int d = 0; d < 8; ++d) o[h][d] += p * vf[i][d];
-    }
-    // the 8 lanes of a key group hold the same scores: sum over key groups only
-    ls += __shfl_xor(ls, 8, 64);
-    ls += __shfl_xor(ls, 16, 64);
-    ls += __shfl_xor(ls, 32, 64);
-    l[h] = ls;
-#pragma unroll
-    for (int d = 0; d < 8; ++d) {
-      float v = o[h][d];
-      v += __shfl_xor(v, 8, 64);
-      v += __shfl_xor(v, 16, 64);
-      v += __shfl_xor(v, 32, 64);
-      o[h][d] = v;
-    }
-  }
-  if (lane < 8) {
-#pragma unroll
-    for (int h = 0; h < 4; ++h)
-#pragma unroll
-      for (int d = 0; d < 8; ++d) wacc[wv][h][dc * 8 + d] = o[h][d];
-  }
+  for (int h = 0; h < 4; ++h) wacc[wv][h][lane] = o[h];
   if (lane == 0) {
 #pragma unroll
     for (int h = 0; h < 4; ++h) {
@@ -596,7 +597,7 @@ __global__ void __launch_bounds__(256) attn_decode_kernel(AttnArgs a) {
     }
   }
   __syncthreads();
-  // combine the 4 waves: thread (h = tid/64, d = tid%64)
+  // combine the 4 waves: thread (h = tid / 64, d = tid % 64)
   const int h = wv, d = lane;
   float M = -INFINITY;
 #pragma unroll
@@ -609,39 +610,44 @@ __global__ void __launch_bounds__(256) attn_decode_kernel(AttnArgs a) {
     L += wl[w][h] * f;
     O += wacc[w][h][d] * f;
   }
-  float* out = a.part + ((((int64_t)r * a.Hkv + g) * a.max_splits + s) * 4 + h) * 66;
-  out[2 + d] = O;
+  const int head = g * 4 + h;
+  const float gate = reinterpret_cast<const float*>(a.gate)[(int64_t)r * a.H + head];
+  float* dst = reinterpret_cast<float*>(a.out) + (int64_t)r * a.H * 64 + head * 64 + d;
+  if (nsplit == 1) {
+    *dst = O / L * gate;
+    return;
+  }
+  // several splits: device-coherent partials, counted in after every store of the block is
+  // acknowledged (see attn_decode_unit_kernel for why no release / acquire pair is needed)
+  float* part = a.part + ((((int64_t)r * a.Hkv + g) * a.max_splits + s) * 4 + h) * 66;
+  __hip_atomic_store(part + 2 + d, O, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   if (d == 0) {
-    out[0] = M;
-    out[1] = L;
+    __hip_atomic_store(part, M, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(part + 1, L, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-}
-
-// Merge split partials, normalise, round as SDPA output, apply the head gate.
-template <typename T>
-__global__ void __launch_bounds__(256) attn_combine_kernel(AttnArgs a) {
-  const int r = blockIdx.x;
-  if (r >= a.ctl->n_rows) return;
-  const int head = blockIdx.y * 4 + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  const int g = head / 4, h = head % 4;
-  const RowDesc rd = a.rows[r];
-  const int pos = rd.pos;
-  const int lo = a.is_local ? max(0, pos - a.window + 1) : 0;
-  const int nsplit = (pos - lo + 1 + kSplitLen - 1) / kSplitLen;
-  const float* base = a.part + (((int64_t)r * a.Hkv + g) * a.max_splits * 4 + h) * 66;
-  float M = -INFINITY;
-  for (int s = 0; s < nsplit; ++s) M = fmaxf(M, base[(int64_t)s * 4 * 66]);
-  float L = 0.f, O = 0.f;
-  for (int s = 0; s < nsplit; ++s) {
-    const float* p = base + (int64_t)s * 4 * 66;
-    const float f = expf(p[0] - M);
-    L += p[1] * f;
-    O += p[2 + lane] * f;
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int32_t* cnt = a.split_done + (int64_t)r * a.Hkv + g;
+    const int prev = __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    s_last = prev == nsplit - 1;
+    if (s_last) __hip_atomic_store(cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  const float o = rnd<T>(O / L);
-  const float gate = to_f(reinterpret_cast<const T*>(a.gate)[(int64_t)r * a.H + head]);
-  reinterpret_cast<T*>(a.out)[(int64_t)r * a.H * 64 + head * 64 + lane] = from_f<T>(o * gate);
+  __syncthreads();
+  if (!s_last) return;
+  const float* all = a.part + (((int64_t)r * a.Hkv + g) * a.max_splits * 4 + h) * 66;
+  auto at = [&](int i, int k) {
+    return __hip_atomic_load(all + (int64_t)i * 4 * 66 + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  M = -INFINITY;
+  for (int i = 0; i < nsplit; ++i) M = fmaxf(M, at(i, 0));
+  L = O = 0.f;
+  for (int i = 0; i < nsplit; ++i) {
+    const float f = expf(at(i, 0) - M);
+    L += at(i, 1) * f;
+    O += at(i, 2 + d) * f;
+  }
+  *dst = O / L * gate;
 }
 
 // ---------------------------------------------------------------------------
@@ -2293,9 +2299,7 @@ int launch_attn_decode(const AttnArgs& a, int dtype, int max_rows, hipStream_t s
     PULSAR_LAUNCH_CHECK();
     return PULSAR_OK;
   }
-  attn_decode_kernel<float><<<dim3(max_rows, a.Hkv, a.max_splits), 256, 0, s>>>(a);
-  PULSAR_LAUNCH_CHECK();
-  attn_combine_kernel<float><<<dim3(max_rows, a.H / 4), 256, 0, s>>>(a);
+  attn_rows_f32_kernel<<<dim3(max_rows, a.Hkv, a.max_splits), 256, 0, s>>>(a);
   PULSAR_LAUNCH_CHECK();
   return PULSAR_OK;
 }
@@ -2320,7 +2324,17 @@ int launch_attn_prefill(const AttnArgs& a, int dtype, int B, hipStream_t s) {
     PULSAR_LAUNCH_CHECK();
     return PULSAR_OK;
   }
-  PULSAR_DISPATCH(dtype, attn_prefill_kernel, dim3(B * ntile, a.Hkv), 256, a);
+  // fp32 prompts whose keys fit one 256-key block take the row-wise kernel (128 tokens: 124 us
+  // in 64-query tiles, 8 workgroups of a long chain each; 11 row-wise); the rule is the prompt's
+  // length alone, so a sequence gets the same arithmetic in any batch
+  if (a.prefill_T <= kSplitLen) {
+    attn_rows_f32_kernel<<<dim3((unsigned)(B * a.prefill_T), a.Hkv), 256, 0, s>>>(a);
+    PULSAR_LAUNCH_CHECK();
+    return PULSAR_OK;
+  }
+  attn_prefill_kernel<float><<<dim3(B * ntile, a.Hkv), 256, 0, s>>>(a);
+  PULSAR_LAUNCH_CHECK();
+  return PULSAR_OK;
 }
 int launch_router_decode(const RouterArgs& a, int dtype, int max_rows, hipStream_t s) {
   PULSAR_DISPATCH(dtype, router_decode_kernel, dim3(max_rows), 256, a);
