@@ -9,6 +9,11 @@ constexpr int kMaxLayers = 16;
 constexpr int kMaxPulses = 3;
 constexpr int kHeadDim = 64;
 constexpr int kPage = 64;  // positions per KV page
+// Ints between the row counts of two experts: a cache line each. Every routed row adds to its
+// experts' counts with an atomic, and the counts of all experts in one line took those of 320
+// rows one after another (router 8.6 us at 320 rows, 6.8 with a line each; 4.7 at 80 rows, where the
+// launch itself bounds it).
+constexpr int kCountStride = 32;
 
 // Take n consecutive pages from a KV page pool (pool[0]: pages handed out, pool[1]: spent
 // flag, pool_pages: pool size). Returns the first page, or -1 after setting the spent flag
@@ -98,7 +103,7 @@ struct GemmArgs {
   int m_fixed;             // ROWS_ALL with ctl == nullptr
   const StepCtl* ctl;
   const int32_t* list;        // ROWS_LIST: [groups][list_stride]
-  const int32_t* list_count;  // ROWS_LIST: [groups]
+  const int32_t* list_count;  // ROWS_LIST: [groups], kCountStride apart
   int64_t list_stride;
   int a_div;               // ROWS_LIST: A row = entry / a_div (1 = same as entry)
   // epilogue operands

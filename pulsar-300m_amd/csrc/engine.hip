@@ -55,7 +55,7 @@ struct Engine {
   int32_t* dec_topk = nullptr;     // decode router top-k ids per layer [L][max_rows][K]
   float* maxprob = nullptr;        // early exit: top-1 probability per logits row
   int32_t* exit_counts = nullptr;  // early exit: [B][4] exits per pulse
-  int32_t *lists = nullptr, *list_count = nullptr;      // decode: [L][E][max_rows*K], [L][E]
+  int32_t *lists = nullptr, *list_count = nullptr;      // decode: [L][E][max_rows*K], [L][E] (kCountStride apart)
   int32_t *p_lists = nullptr, *p_lcount = nullptr;  // prefill (counts per pulse and layer)
   int32_t* p_ids = nullptr;
   RowDesc* p_rows = nullptr;  // [P][R]
@@ -337,9 +337,9 @@ int create(const PulsarModelDesc& m, const PulsarEngineConfig& c, Engine** out) 
   PULSAR_TRY(x.alloc(&x.part, 4 * std::max<size_t>(MR * 4, (size_t)x.B * 4 * kMaxBlock) * x.Hkv *
                                   x.max_splits * 66));
   PULSAR_TRY(x.alloc(&x.lists, 4 * (size_t)x.L * x.E * MR * x.K));
-  PULSAR_TRY(x.alloc(&x.list_count, 4 * (size_t)x.L * x.E));
+  PULSAR_TRY(x.alloc(&x.list_count, 4 * (size_t)x.L * x.E * kCountStride));
   PULSAR_TRY(x.alloc(&x.p_lists, 4 * (size_t)x.E * R * x.K));
-  PULSAR_TRY(x.alloc(&x.p_lcount, 4 * (size_t)x.E * x.L * x.P));
+  PULSAR_TRY(x.alloc(&x.p_lcount, 4 * (size_t)x.E * x.L * x.P * kCountStride));
   PULSAR_TRY(x.alloc(&x.p_ids, 4 * (size_t)x.B * c.max_prompt));
   PULSAR_TRY(x.alloc(&x.p_rows, sizeof(RowDesc) * x.P * (size_t)x.B * c.max_prompt));
   PULSAR_TRY(x.alloc(&x.p_ctl, sizeof(StepCtl) * x.P));
@@ -384,7 +384,7 @@ int create(const PulsarModelDesc& m, const PulsarEngineConfig& c, Engine** out) 
   PULSAR_CHECK_HIP(hipMemset(x.ctl, 0, sizeof(StepCtl)));
   PULSAR_CHECK_HIP(hipMemset(x.last_ctl, 0, sizeof(StepCtl)));
   PULSAR_CHECK_HIP(hipMemset(x.state, 0, sizeof(SeqState) * x.B));
-  PULSAR_CHECK_HIP(hipMemset(x.list_count, 0, 4 * (size_t)x.L * x.E));
+  PULSAR_CHECK_HIP(hipMemset(x.list_count, 0, 4 * (size_t)x.L * x.E * kCountStride));
   PULSAR_CHECK_HIP(hipStreamCreateWithFlags(&x.capture_stream, hipStreamNonBlocking));
   kv_desc(x);
   *out = guard.release();
@@ -566,7 +566,7 @@ int enqueue_pass(Engine& e, const StepCtl* ctl, const RowDesc* rows, const AttnU
     ra.topk_idx = e.dec_topk + (int64_t)l * MR * e.K;
     ra.topk_w = e.topk_w;
     ra.lists = e.lists + (int64_t)l * e.E * lstride;
-    ra.list_count = e.list_count + (int64_t)l * e.E;
+    ra.list_count = e.list_count + (int64_t)l * e.E * kCountStride;
     ra.list_stride = lstride;
     ra.norm_w = m.mlp_norm[l];
     ra.xn = e.xn;
@@ -967,7 +967,7 @@ int prefill(Engine& e, const int32_t* host_ids, int Bq, int T, hipStream_t s) {
                                   hipMemcpyHostToDevice, s));
   PULSAR_CHECK_HIP(hipMemsetAsync(e.ctl, 0, sizeof(StepCtl), s));
   // kept rows per expert of every (pulse, layer)
-  PULSAR_CHECK_HIP(hipMemsetAsync(e.p_lcount, 0, 4 * (size_t)e.E * e.L * e.P, s));
+  PULSAR_CHECK_HIP(hipMemsetAsync(e.p_lcount, 0, 4 * (size_t)e.E * e.L * e.P * kCountStride, s));
 
   PULSAR_TRY(launch_prefill_stem(e.p_ids, m.tok_emb, m.anchor_norm, m.conv_w, e.xn, e.e_state,
                                  Bq, T, D, m.rms_eps, dt, s));
@@ -1108,7 +1108,7 @@ int prefill(Engine& e, const int32_t* host_ids, int Bq, int T, hipStream_t s) {
       // an expert keeps at most C tokens of each sequence
       const int list_max = (int)std::min<long>(BT, (long)Bq * C);
       const int list_avg = std::max(1, (int)((int64_t)BT * e.K / e.E));
-      int32_t* lcount = e.p_lcount + (size_t)(k * e.L + l) * e.E;
+      int32_t* lcount = e.p_lcount + (size_t)(k * e.L + l) * e.E * kCountStride;
       PULSAR_TRY(launch_prefill_capacity(e.topk_idx, e.topk_w, e.keep, e.p_lists, lcount,
                                          lstride, Bq, T, e.K, e.E, C, s));
       g = gemm_base(e);
@@ -1632,10 +1632,18 @@ int pulsar_engine_read(void* handle, int32_t what, void* host_dst, int64_t bytes
       src = e.last_ctl;
       cap = sizeof(StepCtl);
       break;
-    case PULSAR_BUF_EXPERT_COUNTS:
-      src = e.list_count;
-      cap = 4ll * e.L * e.E;
-      break;
+    case PULSAR_BUF_EXPERT_COUNTS: {  // one counter per cache line there, packed here
+      PULSAR_REQUIRE(bytes <= 4ll * e.L * e.E, "engine_read: more bytes than the buffer holds");
+      const size_t n = (size_t)bytes / 4, rest = (size_t)bytes % 4;
+      if (n)
+        PULSAR_CHECK_HIP(hipMemcpy2DAsync(host_dst, 4, e.list_count, 4 * kCountStride, 4, n,
+                                          hipMemcpyDeviceToHost, stream));
+      if (rest)
+        PULSAR_CHECK_HIP(hipMemcpyAsync((char*)host_dst + 4 * n, e.list_count + n * kCountStride,
+                                        rest, hipMemcpyDeviceToHost, stream));
+      PULSAR_CHECK_HIP(hipStreamSynchronize(stream));
+      return PULSAR_OK;
+    }
     case PULSAR_BUF_EXIT_COUNTS:
       src = e.exit_counts;
       cap = 16ll * e.B;

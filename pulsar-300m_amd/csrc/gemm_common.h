@@ -13,9 +13,12 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kXcds = 8;  // MI355X: consecutive workgroups go to the 8 XCDs in turn
 
+// One output. pre: the residual value (EPI_RESID) or the gate column's bias (EPI_QKVG), loaded
+// by the caller.
 template <typename T>
 __device__ __forceinline__ void epilogue(const GemmArgs& g, int epi, int group, void* Cv,
-                                         int64_t ldc, int crow, int col, float acc, float acc_up) {
+                                         int64_t ldc, int crow, int col, float acc, float acc_up,
+                                         float pre) {
   T* C = reinterpret_cast<T*>(Cv);
   switch (epi) {
     case EPI_STORE:
@@ -25,17 +28,13 @@ __device__ __forceinline__ void epilogue(const GemmArgs& g, int epi, int group, 
       if (col < g.n_main) {
         C[(int64_t)crow * ldc + col] = from_f<T>(acc);
       } else {
-        const int h = col - g.n_main;
-        const T* b = reinterpret_cast<const T*>(g.bias) + (int64_t)group * g.bias_group_stride;
-        const float v = rnd<T>(acc + to_f(b[h]));
-        reinterpret_cast<T*>(g.C2)[(int64_t)crow * g.ldc2 + h] = from_f<T>(sigmoidf_(v));
+        const float v = rnd<T>(acc + pre);
+        reinterpret_cast<T*>(g.C2)[(int64_t)crow * g.ldc2 + col - g.n_main] = from_f<T>(sigmoidf_(v));
       }
       break;
-    case EPI_RESID: {
-      T* p = C + (int64_t)crow * ldc + col;
-      *p = from_f<T>(to_f(*p) + rnd<T>(acc));
+    case EPI_RESID:
+      C[(int64_t)crow * ldc + col] = from_f<T>(pre + rnd<T>(acc));
       break;
-    }
     case EPI_SWIGLU: {
       const float gt = rnd<T>(acc), up = rnd<T>(acc_up);
       C[(int64_t)crow * ldc + col] = from_f<T>(gt * sigmoidf_(gt) * up);
@@ -98,7 +97,7 @@ __device__ __forceinline__ int group_rows(const GemmArgs& g, int group) {
   if constexpr (MODE == ROWS_LOGITS) return g.ctl->n_lrows;
   if constexpr (MODE == ROWS_LIST) {
     // the fused all-rows group (-1) exists only in launches with a step control block
-    return group >= 0 ? g.list_count[group] : g.ctl->n_rows;
+    return group >= 0 ? g.list_count[group * kCountStride] : g.ctl->n_rows;
   }
   return g.ctl ? g.ctl->n_rows : g.m_fixed;
 }
@@ -153,7 +152,10 @@ __device__ __forceinline__ void epilogue4(const GemmArgs& g, int epi, int group,
     default:  // EPI_QKVG: q/k/v columns stored, gate columns through the scalar epilogue
       if (col0 >= g.n_main) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) epilogue<bf16>(g, epi, group, Cv, ldc, crow, col0 + j, v[j], 0.f);
+        for (int j = 0; j < 4; ++j)
+          epilogue<bf16>(g, epi, group, Cv, ldc, crow, col0 + j, v[j], 0.f,
+                         to_f(reinterpret_cast<const bf16*>(
+                             g.bias)[(int64_t)group * g.bias_group_stride + col0 + j - g.n_main]));
         return;
       }
 #pragma unroll

@@ -24,7 +24,7 @@ __device__ int resolve_rows(const GemmArgs& g, int group, int tile, int* a_row, 
         break;
       }
       case ROWS_LIST:
-        n = g.list_count[group] - tile * 32;
+        n = g.list_count[group * kCountStride] - tile * 32;
         break;
       case ROWS_ALL: {
         const int tot = g.ctl ? g.ctl->n_rows : g.m_fixed;
@@ -69,6 +69,19 @@ __device__ int resolve_rows(const GemmArgs& g, int group, int tile, int* a_row, 
   return n;
 }
 
+// What an output's epilogue reads: the residual value, or a gate column's bias.
+template <int EPI>
+__device__ __forceinline__ float epilogue_operand(const GemmArgs& g, int group, const void* C,
+                                                  int64_t ldc, int crow, int col) {
+  if constexpr (EPI == EPI_RESID)
+    return reinterpret_cast<const float*>(C)[(int64_t)crow * ldc + col];
+  if constexpr (EPI == EPI_QKVG)
+    return col < g.n_main ? 0.f
+                          : reinterpret_cast<const float*>(
+                                g.bias)[(int64_t)group * g.bias_group_stride + col - g.n_main];
+  return 0.f;
+}
+
 // A few rows: 4 waves per workgroup, one output column per wave, 32-row tile. The wave's
 // weights (K up to 256 KI) go out as soon as the row count is known and stay in registers for
 // every row; the row entries are loaded behind them, one per lane, and broadcast, and two
@@ -92,7 +105,7 @@ __global__ void __launch_bounds__(256) gemm_f32_kernel(GemmArgs g) {
       cnt = g.ctl->pulse_count[group];
       first = g.ctl->pulse_start[group];
       break;
-    case ROWS_LIST: cnt = g.list_count[group]; break;
+    case ROWS_LIST: cnt = g.list_count[group * kCountStride]; break;
     case ROWS_ALL: cnt = g.ctl ? g.ctl->n_rows : g.m_fixed; break;
     case ROWS_LOGITS: cnt = g.ctl->n_lrows; break;
   }
@@ -124,6 +137,10 @@ __global__ void __launch_bounds__(256) gemm_f32_kernel(GemmArgs g) {
     const int r2 = min(r + 1, n - 1);
     const float* a0 = A + (int64_t)__builtin_amdgcn_readlane(arow, r) * lda + lane * 4;
     const float* a1 = A + (int64_t)__builtin_amdgcn_readlane(arow, r2) * lda + lane * 4;
+    const int c0 = __builtin_amdgcn_readlane(entry, r) + g.c_row_offset;
+    const int c1 = __builtin_amdgcn_readlane(entry, r2) + g.c_row_offset;
+    const float p0 = epilogue_operand<EPI>(g, group, Cout, ldc, c0, col);
+    const float p1 = epilogue_operand<EPI>(g, group, Cout, ldc, c1, col);
     float s[2] = {0.f, 0.f}, u[2] = {0.f, 0.f};
     auto dot = [](const f32x4_t& a, const f32x4_t& b) {
       return a[0] * b[0] + a[1] * b[1] + a[2] * b[2] + a[3] * b[3];
@@ -163,10 +180,8 @@ __global__ void __launch_bounds__(256) gemm_f32_kernel(GemmArgs g) {
       s[q] = wave_sum(s[q]);
       if constexpr (kPair) u[q] = wave_sum(u[q]);
     }
-    const int c0 = __builtin_amdgcn_readlane(entry, r) + g.c_row_offset;
-    const int c1 = __builtin_amdgcn_readlane(entry, r2) + g.c_row_offset;
-    if (lane == 0) epilogue<float>(g, EPI, group, Cout, ldc, c0, col, s[0], u[0]);
-    if (lane == 1 && r + 1 < n) epilogue<float>(g, EPI, group, Cout, ldc, c1, col, s[1], u[1]);
+    if (lane == 0) epilogue<float>(g, EPI, group, Cout, ldc, c0, col, s[0], u[0], p0);
+    if (lane == 1 && r + 1 < n) epilogue<float>(g, EPI, group, Cout, ldc, c1, col, s[1], u[1], p1);
   }
 }
 
@@ -261,7 +276,8 @@ __global__ void __launch_bounds__(256, 2) gemm_f32_tile_kernel(GemmArgs g) {
       v += red[w][t][u][j][l];
       if constexpr (kPair) up += red[w][t][u + 2][j][l];
     }
-    epilogue<float>(g, EPI, group, g.C, g.ldc, c_row[row], col0 + c, v, up);
+    epilogue<float>(g, EPI, group, g.C, g.ldc, c_row[row], col0 + c, v, up,
+                    epilogue_operand<EPI>(g, group, g.C, g.ldc, c_row[row], col0 + c));
   }
 }
 

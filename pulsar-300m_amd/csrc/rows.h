@@ -113,7 +113,7 @@ struct PulseInputArgs {
   void* hout_state;         // previous pulse output per state
   void* h_in;
   void* h;
-  int32_t* zero_counts;     // zeroed by block 0 (expert list counts of the step)
+  int32_t* zero_counts;     // zeroed by block 0 (expert list counts of the step, kCountStride apart)
   int n_zero;
   const float* norm_w;      // [P][D] attn_norm of the first layer (nullable)
   void* xn;                 // normed h_in output when norm_w is set
@@ -226,7 +226,7 @@ struct RouterArgs {
   int32_t* topk_idx;   // [rows][K]
   float* topk_w;       // [rows][K] (values rounded through T)
   int32_t* lists;      // [E][list_stride] assignment ids (decode), nullable
-  int32_t* list_count; // [E]
+  int32_t* list_count; // [E], kCountStride apart
   int64_t list_stride;
   const float* norm_w; // norm_router: [P][D] mlp_norm weight
   void* xn;            // norm_router: normed output [rows][D]
@@ -330,7 +330,7 @@ __device__ __forceinline__ void route_topk_fixed(const float* lg, const float* b
     a.topk_idx[(int64_t)r * K + k] = bi[k];
     a.topk_w[(int64_t)r * K + k] = rnd<T>(bs[k] / tot);
     if (a.lists) {
-      const int p = atomicAdd(&a.list_count[bi[k]], 1);
+      const int p = atomicAdd(&a.list_count[bi[k] * kCountStride], 1);
       a.lists[(int64_t)bi[k] * a.list_stride + p] = r * K + k;
     }
   }
@@ -379,7 +379,7 @@ __device__ __forceinline__ void route_topk(const float* lg, int E, int K, const 
     a.topk_idx[(int64_t)r * K + k] = bi[k];
     a.topk_w[(int64_t)r * K + k] = rnd<T>(s[bi[k]] / tot);
     if (a.lists) {
-      const int p = atomicAdd(&a.list_count[bi[k]], 1);
+      const int p = atomicAdd(&a.list_count[bi[k] * kCountStride], 1);
       a.lists[(int64_t)bi[k] * a.list_stride + p] = r * K + k;
     }
   }

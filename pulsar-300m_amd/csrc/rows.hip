@@ -76,7 +76,7 @@ __global__ void __launch_bounds__(64) pulse_input_kernel(PulseInputArgs a) {
   // one wave per row; lane owns elements [lane*EPL, lane*EPL + EPL)
   const int lane = threadIdx.x;
   if (blockIdx.x == 0 && a.zero_counts) {
-    for (int i = lane; i < a.n_zero; i += 64) a.zero_counts[i] = 0;
+    for (int i = lane; i < a.n_zero; i += 64) a.zero_counts[i * kCountStride] = 0;
   }
   const int r = blockIdx.x;
   // the row descriptor is read with the row count (the rows buffer holds a descriptor for
@@ -1652,7 +1652,7 @@ __global__ void __launch_bounds__(256) norm_router_kernel(RouterArgs a) {
     a.topk_idx[o] = lane;
     a.topk_w[o] = rnd<T>(sc / tot);
     if (a.lists) {
-      const int p = atomicAdd(&a.list_count[lane], 1);
+      const int p = atomicAdd(&a.list_count[lane * kCountStride], 1);
       a.lists[(int64_t)lane * a.list_stride + p] = (int)o;
     }
   }
@@ -1980,7 +1980,7 @@ __global__ void __launch_bounds__(256) prefill_select_kernel(
   }
   int tot;
   const int my_off = block_excl_scan_int(mine, s_off, &tot);
-  if (tid == 0) s_base = tot ? atomicAdd(&lcount[e], tot) : 0;
+  if (tid == 0) s_base = tot ? atomicAdd(&lcount[e * kCountStride], tot) : 0;
   __syncthreads();
   int32_t* out = lists + (int64_t)e * list_stride + s_base + my_off;
   if (staged) {
