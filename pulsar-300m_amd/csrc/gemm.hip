@@ -363,34 +363,40 @@ __global__ void __launch_bounds__(64 * kGemmWaves) gemm_bf16_kernel(GemmArgs g) 
 }
 
 // Mid-size row sets (tens to a few hundred rows per group: block verifies, large decode
-// batches). A workgroup of 4 waves owns R = 64 RB rows of one group and CT weight column
-// tiles of 16 (CT = 4: 64 output columns, SwiGLU 32 gate columns and their 32 up twins;
-// CT = 8: twice that); wave w computes rows 16 RB w .. 16 RB (w + 1) - 1 against all CT
-// tiles. The weight tiles of each 32-wide k step go through a ring of S LDS buffers with
-// direct global-to-LDS loads (each wave fetches CT / 4 of the 1 KB tiles, all 4 waves read
-// all CT); the wave's own rows go through the same ring (one 1 KB direct load per 16-row
-// block, read back by the wave alone: 320-row verify 3.15 -> 3.06 ms against loading them
-// into registers, whose 16 lanes of a load touched 16 rows). The launch moves rows x (weight rows) x K x 2 (1/(16 CT) + 1/R) bytes from L2 to
-// the CUs, which bounds it (about 10 TB/s measured: timing copies without the k loop or
-// without the products put the 320-row verify's routed gate/up at 6.2 and 22.9 of its
-// 22.7 us, and rings of 4 to 10 buffers or 2 to 4 k tiles per stage ran alike; lanes past
-// the row count re-read the last row, whose lines their wave's load fetches once). The
-// expert launches take 64 x 128 tiles (RB = 1, CT = 8; 320-row verify: routed gate/up 22.8
-// us in 64 x 64 tiles, 21.1 in 64 x 128, 21.8 in 128 x 128 at one wave per SIMD, 24.4 in
-// 128 x 64) and the attention projections, whose few hundred dense rows need the
-// workgroups, 64 x 64 (RB = 1, CT = 4).
+// batches). A workgroup of 4 waves owns 64 rows of one group and CT weight column tiles of 16
+// (SwiGLU: CT / 2 gate tiles and their up twins); wave w computes rows 16 w .. 16 w + 15
+// against all CT tiles. Two 32-wide k tiles at a time, the weights and the wave's own rows go
+// through a ring of S LDS stages with direct global-to-LDS loads (each wave fetches a quarter
+// of the weights, all 4 read all of them; its rows it reads back alone). What bounds a launch
+// is what a CU streams in: a workgroup moves (64 + 16 CT) x K x 2 bytes, most of them cold, at
+// 30-50 bytes/ns per CU, so the CU with the most of them ends it (timing copies without the k
+// loop or without the products put the 320-row verify's routed gate/up at 6.2 and 22.9 of
+// its then 22.7 us, and rings of more buffers ran alike). The shapes are chosen at
+// launch_mid_shape.
 //
 // Summation order: K is cut into the 8 chunks of gemm_bf16_kernel (wave w of that kernel
 // takes k tiles p K/32 + w KITER + i, pass p, i < KITER), each chunk summed by one chain
 // of matrix-core products from zero and the chunks added in order 0..7 to a zero start,
 // as that kernel's LDS reduction does: the two kernels give identical results, so a
 // caller picks either one by speed alone.
-constexpr int kMidWaves = 4;
+constexpr int kMidWaves = 4, kMidTileRows = 16 * kMidWaves;
+
+// A mid-size tile: kMidTileRows rows and CT weight column tiles of 16, a ring of S stages.
+template <int CT_, int S_>
+struct MidShape {
+  static constexpr int CT = CT_, S = S_;
+  static constexpr int kStage = (2 * CT + 2 * kMidWaves) * 64;  // 16-byte chunks of a stage
+  static constexpr int kLds = S * kStage;
+  static_assert(CT % 2 == 0, "4 waves share the 2 CT weight loads of a stage");
+  // output columns of a column block
+  template <int EPI>
+  static constexpr int columns() { return EPI == EPI_SWIGLU ? CT * 8 : CT * 16; }
+};
 
 // Tile of a 1-D mid-size launch: the tiles that hold rows, ordered (group, row tile,
-// column block) with column blocks fastest and the fused all-rows group (has_g0) first,
-// are cut into 8 contiguous ranges, one per XCD, as in wide_tile.
-template <int MODE, int CW, int R>
+// column block) with column blocks fastest and the fused all-rows group (has_g0, tiles of
+// shape T0) first, are cut into 8 contiguous ranges, one per XCD, as in wide_tile.
+template <int MODE, int EPI, class T, class T0>
 __device__ __forceinline__ bool mid_tile(const GemmArgs& g, int& cb, int& group, int& rt,
                                          int& cnt) {
   const int L = (int)blockIdx.x, xcd = L % kXcds, slot = L / kXcds;
@@ -399,10 +405,11 @@ __device__ __forceinline__ bool mid_tile(const GemmArgs& g, int& cb, int& group,
   const int ng = g.grid_y + s0;  // at most 64 (host check)
   int rows = 0, nx = 0, items = 0;
   if (lane < ng) {
-    const int grp = lane < s0 ? -1 : lane - s0 + g.group_offset;
-    rows = group_rows<MODE>(g, grp);
-    nx = ((lane < s0 ? g.N0 : g.N) + CW - 1) / CW;
-    items = min((rows + R - 1) / R, g.grid_z) * nx;
+    const bool z = lane < s0;
+    rows = min(group_rows<MODE>(g, z ? -1 : lane - s0 + g.group_offset), g.grid_z);
+    nx = z ? (g.N0 + T0::template columns<EPI>() - 1) / T0::template columns<EPI>()
+           : (g.N + T::template columns<EPI>() - 1) / T::template columns<EPI>();
+    items = (rows + kMidTileRows - 1) / kMidTileRows * nx;
   }
   int total = 0;
   for (int j = 0; j < ng; ++j) total += __builtin_amdgcn_readlane(items, j);
@@ -424,185 +431,179 @@ __device__ __forceinline__ bool mid_tile(const GemmArgs& g, int& cb, int& group,
   return false;
 }
 
-// The k loop of one mid-size tile: PASSES passes of 8 KITER k tiles, visited chunk by chunk
-// (chunk w: tiles p 8 KITER + w KITER + i, p < PASSES, i < KITER). wsrc[h]: the wave's
-// weight tile h (tile wv + 4 h of the block) at k tile 0, lane offset included; arow: the
-// wave's A rows at k 0 (lane offset included). tot: the chunk sums added in chunk
-// order.
-template <int KITER, int PASSES, int RB, int CT, int SR>
-__device__ __forceinline__ void mid_kloop(const bf16* const (&wsrc)[CT / 4],
-                                          const bf16* const (&arow)[RB], bf16x8_t (*sW)[CT][64],
-                                          bf16x8_t (*sA)[kMidWaves * RB][64], int aslot, int wv,
-                                          int lane, f32x4_t (&tot)[RB][CT]) {
-  constexpr int CK = KITER * PASSES, STEPS = 8 * CK, KB = 8 * KITER;
-  constexpr int S = SR < STEPS ? SR : STEPS;  // ring buffers in use (at most sW's SR)
-  static_assert(S >= 2, "ring of at least 2 buffers");
-  constexpr int LOADS = CT / 4 + RB;  // vector loads of one wave per step
-  static_assert((S - 2) * LOADS <= 63, "vmcnt range");
-  // k tile of step t of the chunk-ordered sequence
-  auto ktile = [](int t) { return ((t % CK) / KITER) * KB + (t / CK) * KITER + (t % CK) % KITER; };
-  const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
-  f32x4_t acc[RB][CT];
-#pragma unroll
-  for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-    for (int c = 0; c < CT; ++c) tot[rb][c] = zero;
-  auto fetch = [&](int j) {
-    const int kt = ktile(j);
-#pragma unroll
-    for (int h = 0; h < CT / 4; ++h)
-      load_lds16(wsrc[h] + (int64_t)kt * 512, &sW[j % S][wv + 4 * h][0]);
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb) load_lds16(arow[rb] + kt * 32, &sA[j % S][wv * RB + rb][0]);
-  };
-#pragma unroll
-  for (int j = 0; j < S - 1; ++j) fetch(j);
-#pragma unroll
-  for (int s = 0; s < STEPS; ++s) {
-    // steps stay in program order (the scheduler would otherwise keep several chunks'
-    // accumulators live at once)
-    __builtin_amdgcn_sched_barrier(0);
-    // step s's loads are done once at most the S - 2 younger steps' loads are
-    // outstanding; the barrier publishes every wave's weight tiles of step s and retires
-    // step s - 1, whose buffer the next fetch fills
-    if (s + S - 2 < STEPS)
-      wait_vmcnt<(S - 2) * LOADS>();
-    else
-      wait_vmcnt<0>();
-    lds_barrier();
-    if (s + S - 1 < STEPS) fetch(s + S - 1);
-    bf16x8_t fw[CT], xa[RB];
-#pragma unroll
-    for (int c = 0; c < CT; ++c) fw[c] = sW[s % S][c][lane];
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb) xa[rb] = sA[s % S][wv * RB + rb][aslot];
-    // a chunk's chain starts from zero
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-      for (int c = 0; c < CT; ++c)
-        acc[rb][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[rb], fw[c],
-                                                            s % CK == 0 ? zero : acc[rb][c], 0, 0, 0);
-    if ((s + 1) % CK == 0) {
-#pragma unroll
-      for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-        for (int c = 0; c < CT; ++c) tot[rb][c] += acc[rb][c];
-    }
-  }
-}
-
-template <int EPI, int MODE, int KITER, int KMUL0, int RB, int CT, int S>
-__global__ void __launch_bounds__(64 * kMidWaves, 2) gemm_bf16_mid_kernel(GemmArgs g) {
+// One mid-size tile of K = PASSES passes of 8 KITER k tiles, visited chunk by chunk (chunk
+// w: tiles p 8 KITER + w KITER + i, p < PASSES, i < KITER). smem: at least T::kLds chunks.
+template <int EPI, int MODE, int KITER, int PASSES, class T>
+__device__ __forceinline__ void mid_block(const GemmArgs& g, int cb, int group, int rt, int cnt,
+                                          bf16x8_t* smem) {
   constexpr bool kPair = (EPI == EPI_SWIGLU);
-  constexpr int CW = kPair ? CT * 8 : CT * 16;  // output columns per column block
-  constexpr int R = kMidWaves * RB * 16;
-  static_assert(CT == 4 || CT == 8, "4 or 8 weight tiles per workgroup");
-  __shared__ bf16x8_t sW[S][CT][64];
-  // each wave's A rows of a k step go through the same ring: 16 rows x 32 k per row block,
-  // chunk (row m, k chunk q) at slot 4 m + (q ^ 2 (m >> 3)): the load's lanes 4 j .. 4 j + 3
-  // fetch row j's 64 contiguous bytes, and the fragment read (lane = row m, chunk kq) is
-  // free of LDS bank conflicts
-  __shared__ bf16x8_t sA[S][kMidWaves * RB][64];
-  int cb, group, rt, cnt;
-  if (!mid_tile<MODE, CW, R>(g, cb, group, rt, cnt)) return;
+  constexpr int CT = T::CT;
+  constexpr int CK = KITER * PASSES, STEPS = 4 * CK, KB = 8 * KITER, KT = 8 * CK;
+  constexpr int S = T::S < STEPS ? T::S : STEPS;  // ring buffers in use
+  static_assert(S >= 2, "ring of at least 2 buffers");
+  constexpr int NW = CT / 2, NA = 2;  // 1 KB loads of one wave per stage
+  static_assert((S - 2) * (NW + NA) <= 63, "vmcnt range");
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int m = lane & 15, kq = lane >> 4;
   const bool g0 = group < 0;
   const int N = g0 ? g.N0 : g.N;
-  const int KT = (g0 ? g.K0 : g.K) / 32;
   const bf16* W = g0 ? reinterpret_cast<const bf16*>(g.W0)
                      : reinterpret_cast<const bf16*>(g.W) + (int64_t)group * g.w_group_stride;
   const bf16* A = reinterpret_cast<const bf16*>(g0 ? g.A0 : g.A);
   const int64_t lda = g0 ? g.lda0 : g.lda;
   void* Cout = g0 ? g.C0 : g.C;
   const int64_t ldc = g0 ? g.ldc0 : g.ldc;
-  // weight tile c of the block: SwiGLU gate tiles (CT/2) cb + c for c < CT/2 and their up
-  // twins N/16 on; otherwise tiles CT cb + c (tiles past N re-read the last one, never
-  // stored). Wave wv fetches tiles wv + 4 h.
-  const bf16* wsrc[CT / 4];
+  // k tile t of the chunk-ordered sequence; a stage's two lie side by side in memory unless
+  // every k tile of a pass is a chunk of its own and there are several passes
+  auto ktile = [](int t) { return ((t % CK) / KITER) * KB + (t / CK) * KITER + (t % CK) % KITER; };
+  constexpr bool kAdjacent = KITER % 2 == 0 || PASSES == 1;
+  // Unit u of a stage's 2 CT weight loads: weight tile u % CT of its k tile u / CT. Weight
+  // tile c of the block: SwiGLU gate tiles (CT/2) cb + c for c < CT/2 and their up twins
+  // N/16 on; otherwise tiles CT cb + c (tiles past N re-read the last one, never stored).
+  // Wave wv takes units wv + 4 i.
+  const bf16* wsrc[NW];
+  int wk[NW];
 #pragma unroll
-  for (int h = 0; h < CT / 4; ++h) {
-    const int c = wv + 4 * h;
+  for (int i = 0; i < NW; ++i) {
+    const int c = (wv + 4 * i) % CT;
+    wk[i] = (wv + 4 * i) / CT;
     int ct;
     if constexpr (kPair)
       ct = (c < CT / 2 ? 0 : N / 16 - CT / 2) + cb * (CT / 2) + c;
     else
       ct = min(cb * CT + c, N / 16 - 1);
-    wsrc[h] = W + ((int64_t)ct * KT * 64 + lane) * 8;
+    wsrc[i] = W + ((int64_t)ct * KT * 64 + lane) * 8 + (kAdjacent ? wk[i] * 512 : 0);
   }
-  // rows of the wave: 16-row block rb holds tile rows 16 (RB wv + rb) + 0..15; lanes past
-  // the count re-read the last row (computed, never stored). Lane l loads row l >> 2 of
-  // the block (its entry is lane (l >> 2)'s), chunk (l & 3) ^ 2 (l >> 5).
-  const int r0 = rt * R + wv * RB * 16;
-  int ent[RB];
-  const bf16* arow[RB];
+  // The wave's 16 rows of a stage are two loads of 8 rows x 64 k: whole 128-byte lines. (One
+  // k tile, half a line, per load had the next stage's load wait on the same line: 320-row
+  // verify, routed gate/up 20.7 -> 18.6 us.) Lane l of load i fetches row 8 i + (l >> 3),
+  // chunk (l & 7) ^ (row >> 1), so that a row's chunk q lies at slot 8 row + (q ^ (row >> 1))
+  // and the fragment reads are free of LDS bank conflicts. Rows past the count re-read the
+  // last row (computed, never stored); lane m's entry is that of the wave's row m.
+  const int r0 = rt * kMidTileRows + wv * 16;
+  const int im = min(r0 + m, cnt - 1);
+  const int ent = entry_fix<MODE>(group, im, entry_load<MODE>(g, group, im));
+  const bf16* asrc[NA];
+  int ak[NA];
 #pragma unroll
-  for (int rb = 0; rb < RB; ++rb) {
-    const int i = min(r0 + rb * 16 + m, cnt - 1);
-    ent[rb] = entry_fix<MODE>(group, i, entry_load<MODE>(g, group, i));
-    const int el = __shfl(ent[rb], lane >> 2, 64);
-    arow[rb] = A + (int64_t)a_row_of<MODE>(g, group, el) * lda + ((lane & 3) ^ ((lane >> 5) << 1)) * 8;
+  for (int i = 0; i < NA; ++i) {
+    const int el = __shfl(ent, 8 * i + (lane >> 3), 64);
+    const int chunk = (lane & 7) ^ (4 * i + (lane >> 4));
+    ak[i] = chunk >> 2;
+    asrc[i] = A + (int64_t)a_row_of<MODE>(g, group, el) * lda + (kAdjacent ? chunk : chunk & 3) * 8;
   }
-  const int aslot = m * 4 + (kq ^ ((m >> 3) << 1));  // this lane's fragment chunk
+  auto column = [&](int c) { return (cb * (kPair ? CT / 2 : CT) + c) * 16 + m; };
+  auto fetch = [&](int j) {
+    bf16x8_t* st = smem + (j % S) * T::kStage;
+    const int k0 = ktile(2 * j), k1 = ktile(2 * j + 1);
+#pragma unroll
+    for (int i = 0; i < NW; ++i)
+      load_lds16(wsrc[i] + (int64_t)(kAdjacent || !wk[i] ? k0 : k1) * 512, st + (wv + 4 * i) * 64);
+#pragma unroll
+    for (int i = 0; i < NA; ++i)
+      load_lds16(asrc[i] + (kAdjacent || !ak[i] ? k0 : k1) * 32,
+                 st + (2 * CT + 2 * wv + i) * 64);
+  };
   // The residual values (the gate columns' bias) the epilogue reads go out ahead of the k loop:
   // loads and stores may alias as far as the compiler knows, so in the epilogue each of a
   // lane's 16 values waited for its load before the next one's went out (320-row verify: wo
   // 11.4 -> 9.7 us). D layout of 16x16 MFMA: lane holds rows 4 kq + j of its block, column m;
   // the C row of block row r is the entry held by lane r.
   constexpr int NPRE = EPI == EPI_RESID ? CT : 1;
-  float pre[RB][4][NPRE];
-#pragma unroll
-  for (int rb = 0; rb < RB; ++rb)
+  float pre[4][NPRE] = {};
+  if constexpr (EPI == EPI_RESID) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      pre[rb][j][0] = 0.f;
-      if constexpr (EPI == EPI_RESID) {
-        const int64_t at = (int64_t)(__shfl(ent[rb], kq * 4 + j, 64) + g.c_row_offset) * ldc;
+      const int64_t at = (int64_t)(__shfl(ent, kq * 4 + j, 64) + g.c_row_offset) * ldc;
 #pragma unroll
-        for (int c = 0; c < CT; ++c)
-          pre[rb][j][c] = to_f(reinterpret_cast<const bf16*>(Cout)[at + min((cb * CT + c) * 16 + m, N - 1)]);
-      }
+      for (int c = 0; c < CT; ++c)
+        pre[j][c] = to_f(reinterpret_cast<const bf16*>(Cout)[at + min(column(c), N - 1)]);
     }
+  }
   float gate_bias[EPI == EPI_QKVG ? CT : 1] = {};
   if constexpr (EPI == EPI_QKVG) {
 #pragma unroll
     for (int c = 0; c < CT; ++c) {
-      const int col = min((cb * CT + c) * 16 + m, N - 1);
+      const int col = min(column(c), N - 1);
       if (col >= g.n_main)
         gate_bias[c] = to_f(reinterpret_cast<const bf16*>(
             g.bias)[(int64_t)group * g.bias_group_stride + col - g.n_main]);
     }
   }
-  f32x4_t tot[RB][CT];
-  if (g0 && KMUL0 > 1)
-    mid_kloop<KITER, KMUL0, RB, CT, S>(wsrc, arow, sW, sA, aslot, wv, lane, tot);
-  else
-    mid_kloop<KITER, 1, RB, CT, S>(wsrc, arow, sW, sA, aslot, wv, lane, tot);
+  const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+  f32x4_t acc[CT], tot[CT];
 #pragma unroll
-  for (int rb = 0; rb < RB; ++rb) {
+  for (int c = 0; c < CT; ++c) tot[c] = zero;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int crow = __shfl(ent[rb], kq * 4 + j, 64);
-      if (r0 + rb * 16 + kq * 4 + j >= cnt) continue;
-      if constexpr (kPair) {
+  for (int j = 0; j < S - 1; ++j) fetch(j);
 #pragma unroll
-        for (int c = 0; c < CT / 2; ++c)
-          epilogue<bf16>(g, EPI, group, Cout, ldc, crow + g.c_row_offset,
-                         (cb * (CT / 2) + c) * 16 + m, tot[rb][c][j], tot[rb][c + CT / 2][j], 0.f);
-      } else {
+  for (int s = 0; s < STEPS; ++s) {
+    // stages stay in program order (the scheduler would otherwise keep several chunks'
+    // accumulators live at once)
+    __builtin_amdgcn_sched_barrier(0);
+    // stage s's loads are done once at most the S - 2 younger stages' loads are
+    // outstanding; the barrier publishes every wave's loads of stage s and retires stage
+    // s - 1, whose buffer the next fetch fills
+    if (s + S - 2 < STEPS)
+      wait_vmcnt<(S - 2) * (NW + NA)>();
+    else
+      wait_vmcnt<0>();
+    lds_barrier();
+    if (s + S - 1 < STEPS) fetch(s + S - 1);
+    const bf16x8_t* st = smem + (s % S) * T::kStage;
 #pragma unroll
-        for (int c = 0; c < CT; ++c) {
-          const int col = (cb * CT + c) * 16 + m;
-          if (col < N)
-            epilogue<bf16>(g, EPI, group, Cout, ldc, crow + g.c_row_offset, col, tot[rb][c][j], 0.f,
-                           EPI == EPI_RESID  ? pre[rb][j][NPRE > 1 ? c : 0]
-                           : EPI == EPI_QKVG ? gate_bias[EPI == EPI_QKVG ? c : 0]
-                                             : 0.f);
-        }
+    for (int h = 0; h < 2; ++h) {
+      const int t = 2 * s + h;
+      bf16x8_t fw[CT];
+#pragma unroll
+      for (int c = 0; c < CT; ++c) fw[c] = st[(h * CT + c) * 64 + lane];
+      const bf16x8_t xa = st[(2 * CT + 2 * wv) * 64 + m * 8 + ((4 * h + kq) ^ (m >> 1))];
+      // a chunk's chain starts from zero
+#pragma unroll
+      for (int c = 0; c < CT; ++c)
+        acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa, fw[c], t % CK == 0 ? zero : acc[c], 0,
+                                                         0, 0);
+      if ((t + 1) % CK == 0) {
+#pragma unroll
+        for (int c = 0; c < CT; ++c) tot[c] += acc[c];
       }
     }
   }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int crow = __shfl(ent, kq * 4 + j, 64) + g.c_row_offset;
+    if (r0 + kq * 4 + j >= cnt) continue;
+    if constexpr (kPair) {
+#pragma unroll
+      for (int c = 0; c < CT / 2; ++c)
+        epilogue<bf16>(g, EPI, group, Cout, ldc, crow, column(c), tot[c][j], tot[c + CT / 2][j],
+                       0.f);
+    } else {
+#pragma unroll
+      for (int c = 0; c < CT; ++c) {
+        if (column(c) < N)
+          epilogue<bf16>(g, EPI, group, Cout, ldc, crow, column(c), tot[c][j], 0.f,
+                         EPI == EPI_RESID  ? pre[j][NPRE > 1 ? c : 0]
+                         : EPI == EPI_QKVG ? gate_bias[EPI == EPI_QKVG ? c : 0]
+                                           : 0.f);
+      }
+    }
+  }
+}
+
+// The groups in tiles of shape T, the fused all-rows group (K0 = KMUL0 K) in shape T0.
+template <int EPI, int MODE, int KITER, int KMUL0, class T, class T0>
+__global__ void __launch_bounds__(64 * kMidWaves, 2) gemm_bf16_mid_kernel(GemmArgs g) {
+  __shared__ bf16x8_t smem[T::kLds > T0::kLds ? T::kLds : T0::kLds];
+  int cb, group, rt, cnt;
+  if (!mid_tile<MODE, EPI, T, T0>(g, cb, group, rt, cnt)) return;
+  if constexpr (MODE == ROWS_LIST) {
+    if (group < 0) {
+      mid_block<EPI, MODE, KITER, KMUL0, T0>(g, cb, group, rt, cnt, smem);
+      return;
+    }
+  }
+  mid_block<EPI, MODE, KITER, 1, T>(g, cb, group, rt, cnt, smem);
 }
 
 template <int EPI, int MODE, int KMUL0, bool EAGER, bool XCD>
@@ -685,42 +686,55 @@ int launch_one(const GemmArgs& a, int groups, int max_rows, hipStream_t s) {
   return PULSAR_OK;
 }
 
-template <int EPI, int MODE, int KMUL0, int RB, int CT, int S>
+template <int EPI, int MODE, int KMUL0, class T, class T0>
 void launch_mid_k(const GemmArgs& a, dim3 grid, hipStream_t s) {
+  constexpr int B = 64 * kMidWaves;
   switch (a.K) {
-    case 256: gemm_bf16_mid_kernel<EPI, MODE, 1, KMUL0, RB, CT, S><<<grid, 64 * kMidWaves, 0, s>>>(a); break;
-    case 512: gemm_bf16_mid_kernel<EPI, MODE, 2, KMUL0, RB, CT, S><<<grid, 64 * kMidWaves, 0, s>>>(a); break;
-    case 1024: gemm_bf16_mid_kernel<EPI, MODE, 4, KMUL0, RB, CT, S><<<grid, 64 * kMidWaves, 0, s>>>(a); break;
-    default: gemm_bf16_mid_kernel<EPI, MODE, 8, KMUL0, RB, CT, S><<<grid, 64 * kMidWaves, 0, s>>>(a); break;
+    case 256: gemm_bf16_mid_kernel<EPI, MODE, 1, KMUL0, T, T0><<<grid, B, 0, s>>>(a); break;
+    case 512: gemm_bf16_mid_kernel<EPI, MODE, 2, KMUL0, T, T0><<<grid, B, 0, s>>>(a); break;
+    case 1024: gemm_bf16_mid_kernel<EPI, MODE, 4, KMUL0, T, T0><<<grid, B, 0, s>>>(a); break;
+    default: gemm_bf16_mid_kernel<EPI, MODE, 8, KMUL0, T, T0><<<grid, B, 0, s>>>(a); break;
   }
 }
 
-// Tile shape of a mid-size launch: expert lists in 64 x 128 tiles, rows of a pulse or all
-// rows (one dense group) in 64 x 64 tiles; rings of 6 buffers.
-template <int EPI, int RB, int CT, int S>
+// Dense launches (rows of a pulse, all rows: one group) take 64 x 32 tiles, which give a few
+// hundred rows enough workgroups (320 rows: QKV 9.5 us in 64 x 64 tiles, 7.6 in 64 x 32;
+// output projection 9.3 and 7.4; 32 x 64 lies within 0.7 us of 64 x 32, 32 x 32 gained 0.3 on the
+// one and lost 1.2 on the other). Expert lists take 64 x 128 (320-row verify: routed gate/up
+// 18.8 us, 256 rows 16.6; 18.6 and 18.8 in 64 x 64, 18.1 and 21.5 in 96 x 64, 17.6 and 22.8 in
+// 96 x 128: rows less evenly spread over the experts); an all-rows group of twice the K takes tiles of half
+// the columns there, or its few tiles of twice the bytes end the launch (routed down 13.8 us
+// in one shape, 12.8 so; 256 rows 12.9 and 11.4).
+using MidDense = MidShape<2, 4>;
+using MidList = MidShape<8, 3>;
+using MidListK2 = MidShape<4, 3>;
+
+template <int EPI>
 int launch_mid_shape(const GemmArgs& a, int groups, int max_rows, hipStream_t s) {
-  constexpr int R = kMidWaves * RB * 16;
-  constexpr int CW = EPI == EPI_SWIGLU ? CT * 8 : CT * 16;
-  const int ncol = EPI == EPI_SWIGLU ? CT * 8 : 16;
-  if (a.N % ncol != 0 || (a.has_g0 && a.N0 % ncol != 0))
+  const bool list = a.row_mode == ROWS_LIST, k2 = a.has_g0 && a.K0 == 2 * a.K;
+  const int cw = list ? MidList::columns<EPI>() : MidDense::columns<EPI>();
+  const int cw0 = k2 ? MidListK2::columns<EPI>() : MidList::columns<EPI>();
+  // SwiGLU blocks pair gate columns with their up twins: whole blocks only
+  if (a.N % (EPI == EPI_SWIGLU ? cw : 16) != 0 ||
+      (a.has_g0 && a.N0 % (EPI == EPI_SWIGLU ? cw0 : 16) != 0))
     return fail(PULSAR_ERR_UNSUPPORTED, "gemm: mid-size tiles need N % 16 == 0 (SwiGLU: a "
                                         "multiple of the column block)");
   GemmArgs ga = a;
   ga.grid_y = groups;
-  ga.grid_z = (max_rows + R - 1) / R;
-  int64_t items = (int64_t)groups * ga.grid_z * ((a.N + CW - 1) / CW);
-  if (a.has_g0) items += (int64_t)ga.grid_z * ((a.N0 + CW - 1) / CW);
+  ga.grid_z = max_rows;
+  const int64_t tiles = ((int64_t)max_rows + kMidTileRows - 1) / kMidTileRows;
+  int64_t items = groups * tiles * ((a.N + cw - 1) / cw);
+  if (a.has_g0) items += tiles * ((a.N0 + cw0 - 1) / cw0);
   if (items > (int64_t)1 << 30) return fail(PULSAR_ERR_INVALID, "gemm: mid-size launch too large");
   const dim3 grid((unsigned)((items + kXcds - 1) / kXcds * kXcds));
-  const bool k2 = a.has_g0 && a.K0 == 2 * a.K;
   switch (a.row_mode) {
-    case ROWS_PULSE: launch_mid_k<EPI, ROWS_PULSE, 1, RB, CT, S>(ga, grid, s); break;
-    case ROWS_ALL: launch_mid_k<EPI, ROWS_ALL, 1, RB, CT, S>(ga, grid, s); break;
+    case ROWS_PULSE: launch_mid_k<EPI, ROWS_PULSE, 1, MidDense, MidDense>(ga, grid, s); break;
+    case ROWS_ALL: launch_mid_k<EPI, ROWS_ALL, 1, MidDense, MidDense>(ga, grid, s); break;
     case ROWS_LIST:
       if (k2)
-        launch_mid_k<EPI, ROWS_LIST, 2, RB, CT, S>(ga, grid, s);
+        launch_mid_k<EPI, ROWS_LIST, 2, MidList, MidListK2>(ga, grid, s);
       else
-        launch_mid_k<EPI, ROWS_LIST, 1, RB, CT, S>(ga, grid, s);
+        launch_mid_k<EPI, ROWS_LIST, 1, MidList, MidList>(ga, grid, s);
       break;
     default: return fail(PULSAR_ERR_INVALID, "gemm: row mode of a mid-size launch");
   }
@@ -740,8 +754,7 @@ int launch_mid(const GemmArgs& a, int groups, int max_rows, hipStream_t s) {
     return fail(PULSAR_ERR_UNSUPPORTED, "gemm: the all-rows group needs K0 = K or 2K");
   if (groups + (a.has_g0 ? 1 : 0) > 64)
     return fail(PULSAR_ERR_UNSUPPORTED, "gemm: mid-size tiles take at most 64 groups");
-  if (a.row_mode == ROWS_LIST) return launch_mid_shape<EPI, 1, 8, 6>(a, groups, max_rows, s);
-  return launch_mid_shape<EPI, 1, 4, 6>(a, groups, max_rows, s);
+  return launch_mid_shape<EPI>(a, groups, max_rows, s);
 }
 
 }  // namespace
