@@ -112,7 +112,7 @@ __global__ void __launch_bounds__(256) rmsnorm_bwd_vec_kernel(const T* __restric
   constexpr int V = kVec<T>;
   __shared__ __attribute__((aligned(16))) float red[4][64 * NC * V];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nch = dim / V;
-  int at[NC];  // element offset of chunk j in its row (chunks past the row re-read the last one as zero)
+  int at[NC];  // element offset of chunk j in its row; chunks past it re-read the last one as zero
   float wt[NC][V], acc[NC][V];
 #pragma unroll
   for (int j = 0; j < NC; ++j) {
@@ -120,7 +120,10 @@ __global__ void __launch_bounds__(256) rmsnorm_bwd_vec_kernel(const T* __restric
     at[j] = min(c, nch - 1) * V;
     ldv<V>(w + at[j], wt[j]);
 #pragma unroll
-    for (int e = 0; e < V; ++e) acc[j][e] = 0.f;
+    for (int e = 0; e < V; ++e) {
+      if (c >= nch) wt[j][e] = 0.f;  // its factor is zero, but the weight may be infinite
+      acc[j][e] = 0.f;
+    }
   }
   const float inv_dim = 1.0f / (float)dim;
   const int64_t step = (int64_t)gridDim.x * 4 * RPI;

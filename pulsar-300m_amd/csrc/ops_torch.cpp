@@ -40,7 +40,20 @@ struct Args {
   }
 };
 
-void check(int rc) {
+struct Unlocked {  // the interpreter lock given up for a scope
+  PyThreadState* state = PyEval_SaveThread();
+  ~Unlocked() { PyEval_RestoreThread(state); }
+};
+
+// The library call, without the interpreter lock (as through ctypes): a launch can wait for
+// room in the queue.
+template <typename F, typename... A>
+void run(F f, A... args) {
+  int rc;
+  {
+    Unlocked scope;
+    rc = f(args...);
+  }
   if (rc != PULSAR_OK) {
     const char* m = pulsar_last_error();
     throw std::runtime_error(m && *m ? m : "pulsar_hip error " + std::to_string(rc));
@@ -88,8 +101,8 @@ PyObject* rmsnorm_forward(const Args& a) {
   const int64_t dim = x.size(-1), rows = dim ? x.numel() / dim : 0;
   Tensor y = like(x), rs = make(x, {rows}, at::kFloat);
   if (rows)
-    check(pulsar_rmsnorm_forward(p(x), p<float>(w), q(y), q<float>(rs), rows, dim, a.f32(2), code(x),
-                                 stream(x)));
+    run(pulsar_rmsnorm_forward, p(x), p<float>(w), q(y), q<float>(rs), rows, dim, a.f32(2), code(x),
+                                 stream(x));
   return pair(y, rs, false);
 }
 
@@ -97,9 +110,9 @@ PyObject* rmsnorm_forward(const Args& a) {
 PyObject* qk_rmsnorm_rope_forward(const Args& a) {
   const Tensor &x = a.t(0), &w = a.t(1), &c = a.t(2), &s = a.t(3);
   Tensor y = make(x, x.sizes()), rs = make(x, {x.numel() / 64}, at::kFloat);
-  check(pulsar_qk_rmsnorm_rope_forward(p(x), a.i64(7), a.i64(8), a.i64(9), a.i64(4), a.i64(5),
+  run(pulsar_qk_rmsnorm_rope_forward, p(x), a.i64(7), a.i64(8), a.i64(9), a.i64(4), a.i64(5),
                                        a.i64(6), 64, p<float>(w), p<float>(c), p<float>(s), q(y),
-                                       q<float>(rs), a.f32(10), code(x), stream(x)));
+                                       q<float>(rs), a.f32(10), code(x), stream(x));
   return pair(y, rs, false);
 }
 
@@ -108,7 +121,7 @@ PyObject* fused_attn_gate_forward(const Args& a) {
   const Tensor &x = a.t(0), &g = a.t(1);
   const int64_t B = x.size(0), H = x.size(1), T = x.size(2), D = x.size(3);
   Tensor o = make(x, {B, T, H * D});
-  check(pulsar_fused_attn_gate_forward(p(x), p<float>(g), q(o), B, H, T, D, code(x), stream(x)));
+  run(pulsar_fused_attn_gate_forward, p(x), p<float>(g), q(o), B, H, T, D, code(x), stream(x));
   return out(o);
 }
 
@@ -116,8 +129,8 @@ PyObject* fused_attn_gate_forward(const Args& a) {
 PyObject* causal_conv1d_k4_forward(const Args& a) {
   const Tensor &x = a.t(0), &w = a.t(1);
   Tensor y = like(x);
-  check(pulsar_causal_conv1d_k4_forward(p(x), p<float>(w), q(y), x.size(0), x.size(1), x.size(2),
-                                        code(x), stream(x)));
+  run(pulsar_causal_conv1d_k4_forward, p(x), p<float>(w), q(y), x.size(0), x.size(1), x.size(2),
+                                        code(x), stream(x));
   return out(y);
 }
 
@@ -128,7 +141,7 @@ PyObject* fused_swiglu_forward(const Args& a) {
   std::vector<int64_t> shape = gu.sizes().vec();
   shape.back() = d;
   Tensor o = make(gu, shape);
-  if (rows) check(pulsar_fused_swiglu_forward(p(gu), q(o), rows, d, code(gu), stream(gu)));
+  if (rows) run(pulsar_fused_swiglu_forward, p(gu), q(o), rows, d, code(gu), stream(gu));
   return out(o);
 }
 
@@ -140,9 +153,9 @@ PyObject* moe_router_topk_forward(const Args& a) {
   Tensor z = make(l, {}, at::kFloat), pm = make(l, {E}, at::kFloat);
   // per-workgroup partial statistics (merged in a fixed order inside the library)
   Tensor ws = make(l, {std::max<int64_t>(1, pulsar_moe_router_workspace_bytes(N, E) / 4)}, at::kFloat);
-  check(pulsar_moe_router_topk_forward_ws(p(l), code(l), p<float>(b), q<int64_t>(idx),
+  run(pulsar_moe_router_topk_forward_ws, p(l), code(l), p<float>(b), q<int64_t>(idx),
                                           q<uint16_t>(w), q<float>(z), q<float>(pm), N, E, K,
-                                          a.f32(3), q<float>(ws), stream(l)));
+                                          a.f32(3), q<float>(ws), stream(l));
   THPObjectPtr r(PyTuple_New(4));
   if (!r) throw python_error();
   const Tensor* o[4] = {&idx, &w, &z, &pm};
@@ -160,8 +173,8 @@ PyObject* moe_dispatch_forward(const Args& a) {
   const int64_t E = a.i64(3), C = a.i64(4);
   const Tensor n = a.opt(5);
   Tensor o = make(x, {E, C, x.size(1)});
-  check(pulsar_moe_dispatch_forward(p(x), p<int64_t>(ti), p<int32_t>(ts), p<int64_t>(n), q(o),
-                                    x.size(0), x.size(1), ti.size(1), E, C, code(x), stream(x)));
+  run(pulsar_moe_dispatch_forward, p(x), p<int64_t>(ti), p<int32_t>(ts), p<int64_t>(n), q(o),
+                                    x.size(0), x.size(1), ti.size(1), E, C, code(x), stream(x));
   return out(o);
 }
 
@@ -172,9 +185,9 @@ PyObject* moe_combine_forward(const Args& a) {
   const int64_t N = ti.size(0), D = eo.size(2);
   Tensor o = make(eo, {N, D});
   if (N)
-    check(pulsar_moe_combine_forward(p(eo), p<int64_t>(ti), p<uint16_t>(w), p<int32_t>(ts), p(sh),
+    run(pulsar_moe_combine_forward, p(eo), p<int64_t>(ti), p<uint16_t>(w), p<int32_t>(ts), p(sh),
                                      q(o), N, D, ti.size(1), eo.size(0), eo.size(1), code(eo),
-                                     stream(eo)));
+                                     stream(eo));
   return out(o);
 }
 
@@ -183,8 +196,8 @@ PyObject* moe_slots_from_order(const Args& a) {
   const Tensor &f = a.t(0), &o = a.t(1);
   const int64_t M = f.numel(), E = a.i64(2);
   Tensor s = make(f, {M}, at::kInt), n = make(f, {E}, at::kLong);
-  check(pulsar_moe_slots_from_order(p<int64_t>(f), p<int64_t>(o), q<int32_t>(s), q<int64_t>(n), M, E,
-                                    a.i64(3), stream(f)));
+  run(pulsar_moe_slots_from_order, p<int64_t>(f), p<int64_t>(o), q<int32_t>(s), q<int64_t>(n), M, E,
+                                    a.i64(3), stream(f));
   return pair(s, n, false);
 }
 
@@ -192,9 +205,10 @@ PyObject* moe_slots_from_order(const Args& a) {
 PyObject* rmsnorm_backward(const Args& a) {
   const Tensor &dy = a.t(0), &x = a.t(1), &w = a.t(2), &rs = a.t(3);
   const int64_t dim = x.size(-1);
-  Tensor dx = like(x), dw = like(a.t(4));  // zeroed by the library
-  check(pulsar_rmsnorm_backward(p(dy), p(x), p<float>(w), p<float>(rs), q(dx), q<float>(dw),
-                                x.numel() / dim, dim, code(x), stream(x)));
+  // the library zeroes the dim gradients that it adds to; a longer weight's others are zero
+  Tensor dx = like(x), dw = a.t(4).numel() == dim ? like(a.t(4)) : at::zeros_like(a.t(4));
+  run(pulsar_rmsnorm_backward, p(dy), p(x), p<float>(w), p<float>(rs), q(dx), q<float>(dw),
+                                x.numel() / dim, dim, code(x), stream(x));
   return pair(dx, dw, true);
 }
 
@@ -203,10 +217,10 @@ PyObject* qk_rmsnorm_rope_backward(const Args& a) {
   const Tensor &dy = a.t(0), &x = a.t(1), &w = a.t(2), &rs = a.t(3), &c = a.t(4), &s = a.t(5);
   const Tensor& dx = a.t(6);
   Tensor dw = like(w);  // zeroed by the library
-  check(pulsar_qk_rmsnorm_rope_backward(p(dy), p(x), a.i64(10), a.i64(11), a.i64(12), q(dx),
+  run(pulsar_qk_rmsnorm_rope_backward, p(dy), p(x), a.i64(10), a.i64(11), a.i64(12), q(dx),
                                         a.i64(13), a.i64(14), a.i64(15), a.i64(7), a.i64(8), a.i64(9),
                                         64, p<float>(w), p<float>(rs), p<float>(c), p<float>(s),
-                                        q<float>(dw), code(x), stream(x)));
+                                        q<float>(dw), code(x), stream(x));
   return pair(dx, dw, true);
 }
 
@@ -216,8 +230,8 @@ PyObject* fused_attn_gate_backward(const Args& a) {
   const int64_t B = x.size(0), H = x.size(1), T = x.size(2);
   Tensor da = like(x), dg = make(x, {B, T, H}, at::kFloat);
   if (da.numel())
-    check(pulsar_fused_attn_gate_backward(p(go), p(x), p<float>(g), q(da), q<float>(dg), B, H, T, 64,
-                                          code(x), stream(x)));
+    run(pulsar_fused_attn_gate_backward, p(go), p(x), p<float>(g), q(da), q<float>(dg), B, H, T, 64,
+                                          code(x), stream(x));
   return pair(da, dg, true);
 }
 
@@ -226,16 +240,16 @@ PyObject* fused_swiglu_backward(const Args& a) {
   const Tensor &d = a.t(0), &gu = a.t(1);
   const int64_t f = a.i64(2), rows = f ? gu.numel() / (2 * f) : 0;
   Tensor o = like(gu);
-  if (rows) check(pulsar_fused_swiglu_backward(p(d), p(gu), q(o), rows, f, code(gu), stream(gu)));
+  if (rows) run(pulsar_fused_swiglu_backward, p(d), p(gu), q(o), rows, f, code(gu), stream(gu));
   return out(o);
 }
 
 // (dout, x, weight) -> [dx, dw]
 PyObject* causal_conv1d_k4_backward(const Args& a) {
   const Tensor &d = a.t(0), &x = a.t(1), &w = a.t(2);
-  Tensor dx = like(x), dw = like(w);  // zeroed by the library
-  check(pulsar_causal_conv1d_k4_backward(p(d), p(x), p<float>(w), q(dx), q<float>(dw), x.size(0),
-                                         x.size(1), x.size(2), code(x), stream(x)));
+  Tensor dx = like(x), dw = w.numel() == 4 * x.size(2) ? like(w) : at::zeros_like(w);
+  run(pulsar_causal_conv1d_k4_backward, p(d), p(x), p<float>(w), q(dx), q<float>(dw), x.size(0),
+                                         x.size(1), x.size(2), code(x), stream(x));
   return pair(dx, dw, true);
 }
 
@@ -245,9 +259,9 @@ PyObject* moe_router_topk_backward(const Args& a) {
   const Tensor dz = a.opt(4), dp = a.opt(5);
   Tensor o = like(l);
   if (l.size(0))
-    check(pulsar_moe_router_topk_backward(p<uint16_t>(dw), p(l), code(l), p<int64_t>(ti), a.f32(3),
+    run(pulsar_moe_router_topk_backward, p<uint16_t>(dw), p(l), code(l), p<int64_t>(ti), a.f32(3),
                                           p<float>(dz), p<float>(dp), q(o), l.size(0), l.size(1),
-                                          ti.size(1), stream(l)));
+                                          ti.size(1), stream(l));
   return out(o);
 }
 
@@ -257,8 +271,8 @@ PyObject* moe_dispatch_backward(const Args& a) {
   const int64_t N = a.i64(3), D = a.i64(4);
   Tensor o = make(d, {N, D});
   if (N)
-    check(pulsar_moe_dispatch_backward(p(d), p<int64_t>(ti), p<int32_t>(ts), q(o), N, D, ti.size(1),
-                                       d.size(0), d.size(1), code(d), stream(d)));
+    run(pulsar_moe_dispatch_backward, p(d), p<int64_t>(ti), p<int32_t>(ts), q(o), N, D, ti.size(1),
+                                       d.size(0), d.size(1), code(d), stream(d));
   return out(o);
 }
 
@@ -267,9 +281,9 @@ PyObject* moe_combine_backward(const Args& a) {
   const Tensor &d = a.t(0), &eo = a.t(1), &ti = a.t(2), &w = a.t(3), &ts = a.t(4);
   const int64_t N = ti.size(0), K = ti.size(1);
   Tensor de = like(eo), dw = make(eo, {N, K}, at::kBFloat16);
-  check(pulsar_moe_combine_backward(p(d), p(eo), p<int64_t>(ti), p<uint16_t>(w), p<int32_t>(ts),
+  run(pulsar_moe_combine_backward, p(d), p(eo), p<int64_t>(ti), p<uint16_t>(w), p<int32_t>(ts),
                                     q(de), q<uint16_t>(dw), N, eo.size(2), K, eo.size(0), eo.size(1),
-                                    code(eo), stream(eo)));
+                                    code(eo), stream(eo));
   return pair(de, dw, true);
 }
 

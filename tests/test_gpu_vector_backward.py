@@ -37,6 +37,27 @@ def test_rmsnorm_backward_chunks(pc, rows, dim, dtype):  # noqa: F811
         _check(dw, ow, torch.float32, "rmsnorm dw")
 
 
+def test_rmsnorm_backward_infinite_weight(pc):  # noqa: F811
+    """Lanes past a row's last chunk add nothing, an infinite weight in that chunk included."""
+    x = torch.rand(5, 520, device="cuda") + 0.5
+    w, dy = torch.ones(520, device="cuda"), torch.ones(5, 520, device="cuda")
+    w[-1] = float("inf")
+    dx, dw = pc.rmsnorm_backward(dy, x, w, torch.ones(5, device="cuda"))
+    assert bool((dx[:, :-1] == -float("inf")).all()), "dx = r w dy - x inf"
+    assert bool(torch.isfinite(dw).all())
+
+
+def test_backward_of_longer_weights(pc):  # noqa: F811
+    """Gradients of weight entries that no column uses are zero."""
+    x, dy = _rand(1, 6, 64, seed=1), _rand(1, 6, 64, seed=2)
+    for _ in range(8):  # freed blocks hold other values
+        torch.full((4096,), 7.0, device="cuda")
+    w = torch.rand(96, device="cuda")
+    assert not pc.rmsnorm_backward(dy, x, w, torch.ones(6, device="cuda"))[1][64:].any()
+    w = torch.rand(96, 4, device="cuda")
+    assert not pc.causal_depthwise_conv1d_k4_backward(dy, x, w)[1][64:].any()
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("B,H,T", [(1, 1, 1), (3, 4, 11), (1, 16, 65), (2, 3, 2100), (70, 16, 1)])
 def test_qk_backward_groups(pc, B, H, T, dtype):  # noqa: F811
