@@ -373,12 +373,10 @@ __global__ void __launch_bounds__(256) norm_rows_kernel(NormArgs a) {
 // QK-norm + RoPE (+YaRN) on q heads, value residual + K-norm + RoPE on kv heads and the
 // cache write. One wave per head vector (lane = element, rotate-half partner = lane^32);
 // a wave takes head hh of RPW consecutive rows, their loads issued before the first
-// reduction (prefill: 8 rows; decode: 1). The value cache is dimension-major: 8 rows of one
+// reduction (many rows: 8; few: 1). The value cache is dimension-major: 8 rows of one
 // sequence at consecutive positions from a multiple of 8 leave each lane 8 adjacent values
-// of its dimension row, stored as one vector (16 x 2048 tokens: 117 us per launch with one
-// row per wave and element stores, 104 with 2 rows, 95 with 8 rows and vector stores).
-// Prefill and fp32 decode; bf16 decode does the same arithmetic inside
-// attn_decode_unit_kernel.
+// of its dimension row, stored as one vector. fp32, and bf16 prompts of few rows (long ones
+// take the kernel below); bf16 decode does the same arithmetic inside attn_decode_unit_kernel.
 // ---------------------------------------------------------------------------
 template <typename T, int RPW>
 __global__ void __launch_bounds__(256) qk_post_kernel(QKPostArgs a) {
@@ -484,6 +482,110 @@ __global__ void __launch_bounds__(256) qk_post_kernel(QKPostArgs a) {
 #pragma unroll
     for (int i = 0; i < RPW; ++i)
       if (keep[i]) Vc[kv_offset_v(a.kv, a.layer, rd[i].seq, g, rd[i].pos, lane)] = from_f<T>(v[i]);
+  }
+}
+
+// The same for bf16 prompts, 8 consecutive rows per wave and 8 lanes per head vector, 16 bytes
+// a lane: one load instead of 8, sums in 3 lane exchanges for all rows together, the rows'
+// rotary angles held for all heads of the wave (q heads w, w + 4 gridDim.y, ..., four in flight,
+// then its kv heads). Values reach their dimension rows through LDS. The sums add in
+// wave_sum's order and squares of bf16 are exact, so results equal the kernel above bit for
+// bit. Bound by memory: 16 x 2048 tokens, 16 + 4 heads, 92 us a launch with 2-byte lanes (8
+// loads and 48 lane exchanges per head and wave for 1 KB), 42 us so (4.6 TB/s).
+__global__ void __launch_bounds__(256) qk_post_rows8_kernel(QKPostArgs a) {
+  __shared__ __attribute__((aligned(16))) bf16 tile[4][8][72];
+  const int n = a.ctl->n_rows;
+  const int r0 = blockIdx.x * 8;
+  if (r0 >= n) return;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, grp = lane >> 3, c = lane & 7;
+  const int H = a.H, Hk = a.Hkv, first = blockIdx.y * 4 + wv, step = 4 * (int)gridDim.y;
+  const bool live = r0 + grp < n;  // rows past n repeat the last one and are not stored
+  const int r = min(r0 + grp, n - 1);
+  const RowDesc rd = a.rows[r];
+  bf16* row = reinterpret_cast<bf16*>(a.qkv) + (int64_t)r * a.ldq + c * 8;
+  float cs[8], sn[8];
+  ldv<8>(a.cos + (int64_t)rd.pos * 32 + (c & 3) * 8, cs);
+  ldv<8>(a.sin + (int64_t)rd.pos * 32 + (c & 3) * 8, sn);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) sn[e] = c < 4 ? -sn[e] : sn[e];
+  auto norm_rope = [&](const uint4& raw, const float (&w)[8], float (&o)[8]) {
+    float x[8];
+    unpackv<bf16>(raw, x);
+    const float qa = (x[0] * x[0] + x[1] * x[1]) + (x[2] * x[2] + x[3] * x[3]);
+    const float qb = (x[4] * x[4] + x[5] * x[5]) + (x[6] * x[6] + x[7] * x[7]);
+    float ss = qa + dpp_mov<0xB1>(qb);
+    ss += dpp_mov<0xB1>(ss);
+    ss += dpp_mov<0x4E>(ss);
+    ss += dpp_mov<0x141>(ss);  // the other four lanes' sum
+    const float inv = 1.0f / sqrtf(ss / 64.0f + a.eps);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = rnd<bf16>(w[e] * (x[e] * inv));
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float p = dpp_mov<0x1B>(dpp_mov<0x141>(x[e]));  // lane ^ 4: the rotation's partner
+      o[e] = __builtin_fmaf(x[e], cs[e], p * sn[e]);
+    }
+  };
+  constexpr int U = 4;
+  for (int h0 = first; h0 < H; h0 += U * step) {
+    uint4 raw[U];
+    float w[U][8];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int h = min(h0 + u * step, H - 1);
+      raw[u] = *reinterpret_cast<const uint4*>(row + h * 64);
+      ldv<8>(a.q_norm + ((int64_t)rd.pulse * H + h) * 64 + c * 8, w[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      float o[8];
+      norm_rope(raw[u], w[u], o);
+      if (live && h0 + u * step < H) stv<8>(row + (h0 + u * step) * 64, o);
+    }
+  }
+  const bool keep = live && !(a.is_local && rd.pos < a.prefill_T - a.window);
+  const int seq0 = __builtin_amdgcn_readfirstlane(rd.seq), pos0 = __builtin_amdgcn_readfirstlane(rd.pos);
+  // 8 rows of one sequence at consecutive positions from a multiple of 8: 8 adjacent elements
+  // of every dimension row
+  const bool vec = (pos0 & 7) == 0 && (!kv_is_local(a.kv, a.layer) || (a.kv.lcap & 7) == 0) &&
+                   __ballot(keep && rd.seq == seq0 && rd.pos == pos0 + grp) == ~0ull;
+  bf16* Kc = reinterpret_cast<bf16*>(a.kv.k[a.layer]);
+  bf16* Vc = reinterpret_cast<bf16*>(a.kv.v[a.layer]);
+  for (int g = first; g < Hk; g += step) {
+    bf16* vfp = reinterpret_cast<bf16*>(a.v_first) + (int64_t)r * Hk * 64 + g * 64 + c * 8;
+    const uint4 kraw = *reinterpret_cast<const uint4*>(row + (H + g) * 64);
+    const uint4 vraw = *reinterpret_cast<const uint4*>(row + (H + Hk + g) * 64);
+    const uint4 fraw = *reinterpret_cast<const uint4*>(vfp);  // layer 0 writes it
+    float w[8], k[8], v[8];
+    ldv<8>(a.k_norm + ((int64_t)rd.pulse * Hk + g) * 64 + c * 8, w);
+    unpackv<bf16>(vraw, v);
+    if (rd.pulse == 0) {
+      if (a.layer == 0) {
+        if (live) *reinterpret_cast<uint4*>(vfp) = vraw;
+      } else {
+        float f[8];
+        unpackv<bf16>(fraw, f);
+        const float lv = a.v_lambda[0];
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          v[e] = rnd<bf16>(rnd<bf16>(rnd<bf16>(1.0f - lv) * v[e]) + rnd<bf16>(lv * f[e]));
+      }
+    }
+    norm_rope(kraw, w, k);
+    if (keep) stv<8>(Kc + kv_offset(a.kv, a.layer, rd.seq, g, rd.pos) + c * 8, k);
+    if (vec) {
+      stv<8>(&tile[wv][grp][c * 8], v);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the wave reads its own slice back
+      float t[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) t[i] = to_f(tile[wv][i][lane]);
+      stv<8>(Vc + kv_offset_v(a.kv, a.layer, seq0, g, pos0, lane), t);
+      asm volatile("" ::: "memory");
+    } else if (keep) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        Vc[kv_offset_v(a.kv, a.layer, rd.seq, g, rd.pos, c * 8 + e)] = from_f<bf16>(v[e]);
+    }
   }
 }
 
@@ -2229,8 +2331,14 @@ int launch_qk_post(const QKPostArgs& a, int dtype, int max_rows, hipStream_t s) 
   const int rpw = max_rows >= kManyRows ? kPostRowsPerWave : 1;
   const dim3 grid((unsigned)((max_rows + rpw - 1) / rpw), (unsigned)((a.H + a.Hkv + 3) / 4));
   if (dtype == PULSAR_BF16) {
-    if (rpw > 1) qk_post_kernel<bf16, kPostRowsPerWave><<<grid, 256, 0, s>>>(a);
-    else qk_post_kernel<bf16, 1><<<grid, 256, 0, s>>>(a);
+    if (rpw == 8 && a.prefill && a.ldq % 8 == 0 && aligned16(a.qkv) && aligned16(a.q_norm) &&
+        aligned16(a.k_norm) && aligned16(a.cos) && aligned16(a.sin) && aligned16(a.v_first)) {
+      // all heads of 8 rows in one workgroup where that fills the chip, else 4 q heads in each
+      const unsigned ny = grid.x >= 1024 ? 1 : (unsigned)((a.H + 3) / 4);
+      qk_post_rows8_kernel<<<dim3(grid.x, ny), 256, 0, s>>>(a);
+    } else {
+      qk_post_kernel<bf16, 1><<<dim3((unsigned)max_rows, grid.y), 256, 0, s>>>(a);
+    }
   } else {
     if (rpw > 1) qk_post_kernel<float, kPostRowsPerWave><<<grid, 256, 0, s>>>(a);
     else qk_post_kernel<float, 1><<<grid, 256, 0, s>>>(a);
