@@ -2331,6 +2331,8 @@ int launch_qk_post(const QKPostArgs& a, int dtype, int max_rows, hipStream_t s) 
   const int rpw = max_rows >= kManyRows ? kPostRowsPerWave : 1;
   const dim3 grid((unsigned)((max_rows + rpw - 1) / rpw), (unsigned)((a.H + a.Hkv + 3) / 4));
   if (dtype == PULSAR_BF16) {
+    // from kManyRows rows on: 32768 rows 92 -> 42 us; one prompt of 517 tokens, one 8-row
+    // wave per SIMD and no more, is faster row by row (prefill 3.29 against 3.31 ms)
     if (rpw == 8 && a.prefill && a.ldq % 8 == 0 && aligned16(a.qkv) && aligned16(a.q_norm) &&
         aligned16(a.k_norm) && aligned16(a.cos) && aligned16(a.sin) && aligned16(a.v_first)) {
       // all heads of 8 rows in one workgroup where that fills the chip, else 4 q heads in each
