@@ -137,6 +137,7 @@ PyObject* causal_conv1d_k4_forward(const Args& a) {
 // (gu, d_ff) -> out
 PyObject* fused_swiglu_forward(const Args& a) {
   const Tensor& gu = a.t(0);
+  TORCH_CHECK(gu.dim() > 0, "gu must have at least one dimension");
   const int64_t d = a.i64(1), rows = d ? gu.numel() / (2 * d) : 0;
   std::vector<int64_t> shape = gu.sizes().vec();
   shape.back() = d;

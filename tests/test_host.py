@@ -265,6 +265,17 @@ def test_op_wrappers_check_operands_before_the_library_is_called(monkeypatch):
         pc.moe_slots_from_order(idx.view(-1).int(), idx.view(-1), E, C)
 
 
+def test_swiglu_forward_refuses_a_scalar():
+    """A 0-dimensional gu has no last dimension to replace: an error, no memory touched (the
+    native half itself refuses it, so a CPU tensor shows it)."""
+    import torch
+
+    import pulsar_cuda as pc
+
+    with pytest.raises(RuntimeError, match="gu must have at least one dimension"):
+        pc._OPS.fused_swiglu_forward(torch.tensor(1.0), 4)
+
+
 def test_kv_cache_bytes_against_the_reference_table():
     """The reference's published unified-cache table (src/infer.py:834-846):
     73.4 MB at 32k; the engine's footprint differs only by the ring's one-block slack, page
