@@ -217,7 +217,8 @@ PyObject* rmsnorm_backward(const Args& a) {
 PyObject* qk_rmsnorm_rope_backward(const Args& a) {
   const Tensor &dy = a.t(0), &x = a.t(1), &w = a.t(2), &rs = a.t(3), &c = a.t(4), &s = a.t(5);
   const Tensor& dx = a.t(6);
-  Tensor dw = like(w);  // zeroed by the library
+  // the library zeroes the H x 64 gradients that it adds to; a wider weight's others are zero
+  Tensor dw = w.numel() == 64 * a.i64(8) ? like(w) : at::zeros_like(w);
   run(pulsar_qk_rmsnorm_rope_backward, p(dy), p(x), a.i64(10), a.i64(11), a.i64(12), q(dx),
                                         a.i64(13), a.i64(14), a.i64(15), a.i64(7), a.i64(8), a.i64(9),
                                         64, p<float>(w), p<float>(rs), p<float>(c), p<float>(s),

@@ -56,6 +56,12 @@ def test_backward_of_longer_weights(pc):  # noqa: F811
     assert not pc.rmsnorm_backward(dy, x, w, torch.ones(6, device="cuda"))[1][64:].any()
     w = torch.rand(96, 4, device="cuda")
     assert not pc.causal_depthwise_conv1d_k4_backward(dy, x, w)[1][64:].any()
+    w, (cos, sin) = torch.rand(2, 1024, device="cuda"), _tables(3)
+    q, dq = x.view(1, 2, 3, 64), dy.view(1, 2, 3, 64)
+    sevens = [torch.full_like(w, 7.0) for _ in range(8)]
+    del sevens
+    dw = pc.qk_rmsnorm_rope_backward(dq, q, w, torch.ones(6, device="cuda"), cos, sin, 3)[1]
+    assert dw.shape == w.shape and not dw.view(-1)[2 * 64:].any()
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
