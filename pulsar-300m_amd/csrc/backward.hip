@@ -433,7 +433,10 @@ __global__ void __launch_bounds__(256) dispatch_bwd_vec_kernel(const T* __restri
   const int64_t t = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (t >= N) return;
   const int nrow = kept_row(idx, slots, t, K, E, C, lane);
-  for (int c = lane * V; c < D; c += 64 * V) {
+  // every lane runs every pass, those past the row re-reading its last chunk: the broadcasts
+  // below read lanes 0 .. K - 1, which a row of fewer chunks than K would have switched off
+  for (int c0 = 0; c0 < D; c0 += 64 * V) {
+    const int c = c0 + lane * V, cl = min(c, D - V);
     float acc[V];
 #pragma unroll
     for (int e = 0; e < V; ++e) acc[e] = 0.f;
@@ -443,7 +446,7 @@ __global__ void __launch_bounds__(256) dispatch_bwd_vec_kernel(const T* __restri
       for (int q = 0; q < 4; ++q) {
         // branch-free: dropped assignments read row 0 and count as zero
         const int at = k0 + q < K ? __builtin_amdgcn_readlane(nrow, k0 + q) : -1;
-        r[q] = *reinterpret_cast<const uint4*>(dei + (int64_t)max(at, 0) * D + c);
+        r[q] = *reinterpret_cast<const uint4*>(dei + (int64_t)max(at, 0) * D + cl);
         if (at < 0) r[q] = make_uint4(0u, 0u, 0u, 0u);
       }
 #pragma unroll
@@ -454,7 +457,7 @@ __global__ void __launch_bounds__(256) dispatch_bwd_vec_kernel(const T* __restri
         for (int e = 0; e < V; ++e) acc[e] += v[e];
       }
     }
-    stv<V>(dx + t * D + c, acc);
+    if (c < D) stv<V>(dx + t * D + c, acc);
   }
 }
 

@@ -128,8 +128,9 @@ def test_conv_backward_leaves_out_terms_past_the_ends(pc, T):  # noqa: F811
 
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("N,D,K", [(1, 8, 1), (5, 520, 3), (33, 1024, 4), (6, 2048, 8),
-                                   (7, 2056, 5)])
+                                   (7, 2056, 5), (9, 8, 4), (5, 24, 8), (6, 1032, 4)])
 def test_moe_backward_chunks(pc, N, D, K, dtype):  # noqa: F811
+    """Rows of whole waves and of less, down to fewer chunks than assignments (D = 8, 24)."""
     E, C = 16, max(2, int(np.ceil(N * K / 16 * 0.9)))
     idx, slots = _routing(N, K, E, C, N)
     ti, ts = torch.as_tensor(idx, device="cuda"), torch.as_tensor(slots, device="cuda")
