@@ -232,6 +232,7 @@ def test_op_wrappers_check_operands_before_the_library_is_called(monkeypatch):
             raise AssertionError(f"library called: {name}")
 
     monkeypatch.setattr(pc, "_LIB", NoLib())
+    monkeypatch.setattr(pc, "_OPS", NoLib())
     monkeypatch.setattr(pc, "_cuda", lambda t, n: None)
     monkeypatch.setattr(pc, "_stream", lambda t: 0)
     E, C, D, N, K = 4, 8, 16, 5, 2
