@@ -232,7 +232,7 @@ enum ProfClass {
   PC_INPUT = 0, PC_NORM, PC_QKVG, PC_QKPOST, PC_ATTN, PC_WO, PC_ROUTER, PC_SHARED_GU,
   PC_ROUTED_GU, PC_SHARED_DOWN, PC_ROUTED_DOWN, PC_COMBINE, PC_OUTPUT, PC_LMHEAD, PC_SAMPLE,
   PC_CONTROL, PC_EVENT_PAIR
-};
+};  // nothing is recorded under PC_OUTPUT: the last MoE combine of a pass does the pulse output
 
 // From kMidRows rows up to kWideRows the projections run in the mid-size tiles of
 // launch_gemm_mid (64-row tiles, weights staged through LDS). They give results
@@ -1189,7 +1189,6 @@ int prefill(Engine& e, const int32_t* host_ids, int Bq, int T, hipStream_t s) {
     po.ctl = ctl;
     po.rows = prow;
     po.D = D;
-    po.prefill = 1;
     po.prefill_T = T;
     po.eps = m.rms_eps;
     po.h_in = e.h_in;

@@ -10,11 +10,12 @@ namespace pulsar {
 
 namespace {
 
-// Resolve the (A row, C row) pairs of this workgroup's 32-row tile into LDS.
+// Resolve the (A row, C row) pairs of this workgroup's 32-row tile into LDS (launches without
+// an all-rows group).
 // Returns the number of valid rows (0 => nothing to do).
 __device__ int resolve_rows(const GemmArgs& g, int group, int tile, int* a_row, int* c_row) {
   __shared__ int s_n;
-  const int mode = (g.has_g0 && group < 0) ? ROWS_ALL : g.row_mode;
+  const int mode = g.row_mode;
   if (threadIdx.x == 0) {
     int n = 0;
     switch (mode) {

@@ -260,8 +260,7 @@ struct CombineArgs {
 struct PulseOutputArgs {
   const StepCtl* ctl;
   const RowDesc* rows;
-  int D, prefill, prefill_T;
-  int slots;                // token-state slots per sequence
+  int D, prefill_T;
   float eps;
   const void* h_in;
   const void* h;

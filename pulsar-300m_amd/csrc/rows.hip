@@ -1786,14 +1786,13 @@ __global__ void __launch_bounds__(256) router_prefill_kernel(RouterArgs a) {
 
 // Prefill router in bf16 on the matrix cores: logits[rows][E] = X . bf16(W)^T with fp32
 // accumulation, E <= 16 experts as the 16 columns of one v_mfma_f32_16x16x32_bf16 tile;
-// a wave owns 16 rows, a workgroup of 8 waves converts the weights into LDS once for its
-// 128 rows (16 x 2048 tokens: 28.1 -> 21.4 us per launch against every wave loading and
-// converting them itself). The logits, rounded to bf16, go through LDS to the shared top-k
+// a wave owns 16 rows, a workgroup converts the weights into LDS once for its 16 RW rows (16 x
+// 2048 tokens, 128 rows: 28.1 -> 21.4 us per launch against every wave loading and converting
+// them itself). The logits, rounded to bf16, go through LDS to the shared top-k
 // routine (one lane per row), so routing is the same as router_prefill_kernel's.
 // All 8 waves stage; waves 0 .. RW - 1 compute, so that a short prompt's rows spread over the
 // CUs. The rows' and the weights' loads all go out before the first is used (KS = D / 32).
 constexpr int kRouterWaves = 8;
-constexpr int kRouterMaxD = 1024;   // model widths the staged weights cover
 template <int KS, int RW>
 __global__ void __launch_bounds__(64 * kRouterWaves) router_prefill_mfma_kernel(RouterArgs a) {
   // the pulse's weights, rounded to bf16 once per workgroup, in B-operand order: k step t,
@@ -2220,7 +2219,8 @@ __global__ void __launch_bounds__(64) moe_combine_rows_kernel(CombineArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// Pulse output (harmonic residual) and, for rows that need logits, the final RMSNorm.
+// Pulse output (harmonic residual) and, for rows that need logits, the final RMSNorm: prefill
+// (decode does it in the last layer's MoE combine).
 // ---------------------------------------------------------------------------
 template <typename T>
 __global__ void __launch_bounds__(256) pulse_output_kernel(PulseOutputArgs a) {
@@ -2229,7 +2229,7 @@ __global__ void __launch_bounds__(256) pulse_output_kernel(PulseOutputArgs a) {
   if (r >= a.ctl->n_rows) return;
   const RowDesc rd = a.rows[r];
   const int D = a.D;
-  const int st = a.prefill ? rd.pos + rd.seq * a.prefill_T : rd.seq * a.slots + rd.sslot;
+  const int st = rd.pos + rd.seq * a.prefill_T;
   const T* hi = reinterpret_cast<const T*>(a.h_in) + (int64_t)r * D;
   const T* h = reinterpret_cast<const T*>(a.h) + (int64_t)r * D;
   const T* rs = reinterpret_cast<const T*>(a.res_scale) + (int64_t)rd.pulse * D;
@@ -2477,7 +2477,6 @@ int launch_norm_router(const RouterArgs& a, int dtype, int max_rows, hipStream_t
 int launch_router_prefill(const RouterArgs& a, int dtype, hipStream_t s) {
   if (a.E > 32) return fail(PULSAR_ERR_UNSUPPORTED, "router: at most 32 experts");
   if (dtype == PULSAR_BF16 && a.E <= 16 && (a.D == 256 || a.D == 512 || a.D == 1024)) {
-    static_assert(kRouterMaxD == 1024, "the widths above");
     if (a.m_fixed <= 0) return PULSAR_OK;
     // 16-row tiles per workgroup: as many as leave a workgroup for every CU (517 rows: 16.5 us
     // at 8 tiles, 5 workgroups; 11.2 at one)

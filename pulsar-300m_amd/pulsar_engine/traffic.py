@@ -68,6 +68,7 @@ def step_bytes(cfg: PulsarConfig, es: int, rows, expert_counts, n_lrows: int,
         out["shared_down"] += D * ds * es + n * (ds + D) * es
         out["routed_down"] += touched * D * de * es + assigned * (de + D) * es
         out["moe_combine"] += n * (K + 3) * D * es
+    # its launch is the last layer's combine: no time is recorded under this class
     out["pulse_output"] = n * 3 * D * es + n_lrows * D * es
     if n_lrows:
         out["lm_head"] = V * D * es + n_lrows * (D * es + V * 4)

@@ -38,7 +38,8 @@ def test_prefill_logits_do_not_depend_on_the_tile_shape(model, T):
 
     # tiles of the widest projection (1552 columns): 128 rows take 64 x 64 tiles, 2000 rows
     # 64 x 128, 4000 rows 128 x 128, 16384 rows and more 128 x 256; attention in 16, 32 and 64
-    # queries; the router in 1, 4 and (260 tokens) 8 row tiles
+    # queries; the router in 1, 4 and (260 tokens) 8 row tiles; q/k norm and RoPE row by row and,
+    # from 1024 rows, 8 rows at a time (across sequences and the window's start)
     sets = {B: logits(B) for B in (1, 16, 32, 128)}
     for B, got in sets.items():
         assert np.isfinite(got).all()
