@@ -400,14 +400,19 @@ GemmArgs gemm_base(const Engine& e) {
 }
 
 // Engines whose steps hold kWideHeadRows rows or more (verify blocks, batches of 64+) run
-// the output head in the LDS tiles of the prefill GEMMs (its 64 MiB of weights read once per
-// 128 rows instead of once per 32); from kWideRows rows (the draft-block
-// mode at batch 256) the decode projections too. Below that the row-tile and mid-size
-// GEMMs are faster: 128 x 256 tiles leave most CUs idle at a few hundred rows (320-row
-// verify: 3.78 against 5.35 ms with every projection in wide tiles). The wide tiles sum K
-// in another order than the row-tile and mid-size kernels (which agree exactly), so an
-// engine's logits can differ from an engine's on the other side of a wide threshold by
-// bf16 rounding; engines on the same side agree exactly.
+// the output head in the LDS tiles of the prefill GEMMs: its 64 MiB of weights are read once
+// per 128 rows (per 64 at 128 rows) instead of once per 32 (128 logits rows: 29 us against 34,
+// 320: 53 against 170). Draft-block engines, most of whose steps hold few of those rows, lose
+// up to 2 % by it below about 640 rows (24 tokens with 240, 360, 642 and 960 rows: 15.95, 16.95,
+// 19.2 and 22.3 ms, without it 15.7, 16.7, 19.1 and 23.1); the reference schedule gains (128, 256
+// and 400 rows: 23.0, 25.3 and 30.2 ms, without it 23.1, 25.5 and 31.1).
+// From kWideRows rows (the draft-block mode from 128 to 256 sequences on, by draft length) the
+// decode projections run in them too. That line was drawn against the row-tile kernel. The
+// mid-size tiles, as they are now, are faster wherever both were timed (24 tokens with 642, 960
+// and 1200 rows: 19.2, 22.3 and 25.3 ms against 26.4, 30.7 and 33.6), so what holds the line is
+// the results alone: the wide tiles sum K in another order than the row-tile and mid-size
+// kernels (which agree exactly), so an engine's logits can differ from an engine's on the other
+// side of a wide threshold by bf16 rounding; engines on the same side agree exactly.
 constexpr int kWideHeadRows = 128;
 constexpr int kWideRows = 1024;
 

@@ -284,7 +284,8 @@ int launch_shape(const GemmArgs& a, int groups, int max_rows, hipStream_t s) {
   return PULSAR_OK;
 }
 
-// The smallest shape whose tiles are at most two per CU, the large one when none is. A CU that
+// The smallest shape whose tiles are at most two per CU, the large one when none is (128 x 128
+// only below two per CU: at exactly two, the last line's 512 rows, the large tile wins). A CU that
 // holds one workgroup streams its operands at 30-50 bytes/ns (outstanding misses), so a launch
 // of few tiles is as slow as one tile's bytes: 128 x 256 x 1024 takes 27 us however few rows
 // there are, 64 x 64 10 us. With every CU busy twice over the larger tile's fewer bytes per
@@ -294,6 +295,8 @@ int launch_shape(const GemmArgs& a, int groups, int max_rows, hipStream_t s) {
 //   wo           1400     12.8 / 14.0 / 18.9 / 28.6   4000  24.6 / 18.8 / 20.4 / 29.6
 //   routed gate/up (rows each of 16 experts) 129      24.1 / 19.5 / 19.7 / 28.0
 //                350      39.0 / 32.7 / 26.8 / 29.8   512   50.8 / 39.3 / 39.9 / 35.3
+// The decode output head (32768 columns) goes by the same rule: 128 rows, exactly two 64 x 128
+// tiles per CU, take 29 us in them and 46 in 128 x 256; more rows take the large tile.
 constexpr int64_t kWideTiles = 512;
 template <int EPI, int MODE>
 int launch_wide(const GemmArgs& a, int groups, int max_rows, hipStream_t s) {
