@@ -814,6 +814,7 @@ int pulsar_rope_forward(const void* x, void* y, const float* cos, const float* s
   PULSAR_REQUIRE(head_dim > 0 && head_dim % 2 == 0, "rope: head_dim must be even");
   PULSAR_REQUIRE(T > 0 || rows == 0, "rope: T must be positive");
   if (rows == 0) return PULSAR_OK;
+  PULSAR_REQUIRE(x && y && cos && sin, "rope: null pointer");
   return dispatch_dtype(dtype, [&](auto tag) {
     using T_ = decltype(tag);
     if ((head_dim / 2) % 8 == 0 && aligned16(x) && aligned16(y) && aligned16(cos) &&

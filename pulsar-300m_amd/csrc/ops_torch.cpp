@@ -66,12 +66,18 @@ hipStream_t stream(const Tensor& t) {
   return c10::hip::getCurrentHIPStream(t.device().index()).stream();
 }
 
-const void* p(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
-void* q(const Tensor& t) { return t.data_ptr(); }
+// A tensor with elements but without memory (a fake one, while a program is traced) is an error
+// here: the kernels would read and write address 0.
+void* q(const Tensor& t) {
+  void* d = t.data_ptr();
+  TORCH_CHECK(d || t.numel() == 0, "the tensor has no memory to read or write");
+  return d;
+}
+const void* p(const Tensor& t) { return t.defined() ? q(t) : nullptr; }
 template <typename X>
 const X* p(const Tensor& t) { return reinterpret_cast<const X*>(p(t)); }
 template <typename X>
-X* q(const Tensor& t) { return reinterpret_cast<X*>(t.data_ptr()); }
+X* q(const Tensor& t) { return reinterpret_cast<X*>(q(t)); }
 
 Tensor like(const Tensor& t) { return at::empty_like(t); }
 Tensor make(const Tensor& on, at::IntArrayRef shape, at::ScalarType dt) {

@@ -6,6 +6,7 @@ from __future__ import annotations
 import csv
 import importlib.util
 import os
+import warnings
 
 import pytest
 
@@ -275,6 +276,24 @@ def test_swiglu_forward_refuses_a_scalar():
 
     with pytest.raises(RuntimeError, match="gu must have at least one dimension"):
         pc._OPS.fused_swiglu_forward(torch.tensor(1.0), 4)
+
+
+def test_ops_refuse_tensors_without_memory():
+    """Fake tensors (shapes only, address 0) raise before any launch: the native half on CPU
+    stand-ins, and the library's RoPE entry for the one op that calls it directly."""
+    import torch
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    import pulsar_cuda as pc
+    from pulsar_cuda import _lib
+
+    with FakeTensorMode() as mode, warnings.catch_warnings():
+        warnings.simplefilter("ignore")  # torch's own, at the pointer's first reading
+        gu = mode.from_tensor(torch.ones(2, 8))
+        with pytest.raises(RuntimeError, match="no memory"):
+            pc._OPS.fused_swiglu_forward(gu, 4)
+    assert pc._LIB.pulsar_rope_forward(None, None, None, None, 2, 2, 64, _lib.PULSAR_F32, None) != 0
+    assert b"null pointer" in pc._LIB.pulsar_last_error()
 
 
 def test_kv_cache_bytes_against_the_reference_table():
