@@ -79,7 +79,25 @@ const X* p(const Tensor& t) { return reinterpret_cast<const X*>(p(t)); }
 template <typename X>
 X* q(const Tensor& t) { return reinterpret_cast<X*>(q(t)); }
 
-Tensor like(const Tensor& t) { return at::empty_like(t); }
+// An output of the layout of argument i. A subclass of torch.Tensor allocates it by its own
+// empty_like, so that it is of the subclass's type.
+Tensor like(const Args& a, int i) {
+  const Tensor& t = a.t(i);
+  if (THPVariable_CheckExact(a.a[i])) return at::empty_like(t);
+  THPObjectPtr torch(PyImport_ImportModule("torch"));
+  if (!torch) throw python_error();
+  THPObjectPtr r(PyObject_CallMethod(torch.get(), "empty_like", "O", a.a[i]));
+  if (!r) throw python_error();
+  TORCH_CHECK_TYPE(THPVariable_Check(r.get()), "empty_like of a tensor subclass gave no tensor");
+  return THPVariable_Unpack(r.get());
+}
+// The gradient of weight argument i. The library zeroes the used entries that it adds to; a
+// longer weight's others are zero too.
+Tensor like_weight(const Args& a, int i, int64_t used) {
+  Tensor dw = like(a, i);
+  if (dw.numel() != used) dw.zero_();
+  return dw;
+}
 Tensor make(const Tensor& on, at::IntArrayRef shape, at::ScalarType dt) {
   return at::empty(shape, on.options().dtype(dt).requires_grad(false));
 }
@@ -105,7 +123,7 @@ PyObject* pair(const Tensor& a, const Tensor& b, bool list) {
 PyObject* rmsnorm_forward(const Args& a) {
   const Tensor &x = a.t(0), &w = a.t(1);
   const int64_t dim = x.size(-1), rows = dim ? x.numel() / dim : 0;
-  Tensor y = like(x), rs = make(x, {rows}, at::kFloat);
+  Tensor y = like(a, 0), rs = make(x, {rows}, at::kFloat);
   if (rows)
     run(pulsar_rmsnorm_forward, p(x), p<float>(w), q(y), q<float>(rs), rows, dim, a.f32(2), code(x),
                                  stream(x));
@@ -134,7 +152,7 @@ PyObject* fused_attn_gate_forward(const Args& a) {
 // (x, weight) -> y
 PyObject* causal_conv1d_k4_forward(const Args& a) {
   const Tensor &x = a.t(0), &w = a.t(1);
-  Tensor y = like(x);
+  Tensor y = like(a, 0);
   run(pulsar_causal_conv1d_k4_forward, p(x), p<float>(w), q(y), x.size(0), x.size(1), x.size(2),
                                         code(x), stream(x));
   return out(y);
@@ -212,8 +230,7 @@ PyObject* moe_slots_from_order(const Args& a) {
 PyObject* rmsnorm_backward(const Args& a) {
   const Tensor &dy = a.t(0), &x = a.t(1), &w = a.t(2), &rs = a.t(3);
   const int64_t dim = x.size(-1);
-  // the library zeroes the dim gradients that it adds to; a longer weight's others are zero
-  Tensor dx = like(x), dw = a.t(4).numel() == dim ? like(a.t(4)) : at::zeros_like(a.t(4));
+  Tensor dx = like(a, 1), dw = like_weight(a, 4, dim);
   run(pulsar_rmsnorm_backward, p(dy), p(x), p<float>(w), p<float>(rs), q(dx), q<float>(dw),
                                 x.numel() / dim, dim, code(x), stream(x));
   return pair(dx, dw, true);
@@ -223,8 +240,7 @@ PyObject* rmsnorm_backward(const Args& a) {
 PyObject* qk_rmsnorm_rope_backward(const Args& a) {
   const Tensor &dy = a.t(0), &x = a.t(1), &w = a.t(2), &rs = a.t(3), &c = a.t(4), &s = a.t(5);
   const Tensor& dx = a.t(6);
-  // the library zeroes the H x 64 gradients that it adds to; a wider weight's others are zero
-  Tensor dw = w.numel() == 64 * a.i64(8) ? like(w) : at::zeros_like(w);
+  Tensor dw = like_weight(a, 2, 64 * a.i64(8));
   run(pulsar_qk_rmsnorm_rope_backward, p(dy), p(x), a.i64(10), a.i64(11), a.i64(12), q(dx),
                                         a.i64(13), a.i64(14), a.i64(15), a.i64(7), a.i64(8), a.i64(9),
                                         64, p<float>(w), p<float>(rs), p<float>(c), p<float>(s),
@@ -236,7 +252,7 @@ PyObject* qk_rmsnorm_rope_backward(const Args& a) {
 PyObject* fused_attn_gate_backward(const Args& a) {
   const Tensor &go = a.t(0), &x = a.t(1), &g = a.t(2);
   const int64_t B = x.size(0), H = x.size(1), T = x.size(2);
-  Tensor da = like(x), dg = make(x, {B, T, H}, at::kFloat);
+  Tensor da = like(a, 1), dg = make(x, {B, T, H}, at::kFloat);
   if (da.numel())
     run(pulsar_fused_attn_gate_backward, p(go), p(x), p<float>(g), q(da), q<float>(dg), B, H, T, 64,
                                           code(x), stream(x));
@@ -247,7 +263,7 @@ PyObject* fused_attn_gate_backward(const Args& a) {
 PyObject* fused_swiglu_backward(const Args& a) {
   const Tensor &d = a.t(0), &gu = a.t(1);
   const int64_t f = a.i64(2), rows = f ? gu.numel() / (2 * f) : 0;
-  Tensor o = like(gu);
+  Tensor o = like(a, 1);
   if (rows) run(pulsar_fused_swiglu_backward, p(d), p(gu), q(o), rows, f, code(gu), stream(gu));
   return out(o);
 }
@@ -255,7 +271,7 @@ PyObject* fused_swiglu_backward(const Args& a) {
 // (dout, x, weight) -> [dx, dw]
 PyObject* causal_conv1d_k4_backward(const Args& a) {
   const Tensor &d = a.t(0), &x = a.t(1), &w = a.t(2);
-  Tensor dx = like(x), dw = w.numel() == 4 * x.size(2) ? like(w) : at::zeros_like(w);
+  Tensor dx = like(a, 1), dw = like_weight(a, 2, 4 * x.size(2));
   run(pulsar_causal_conv1d_k4_backward, p(d), p(x), p<float>(w), q(dx), q<float>(dw), x.size(0),
                                          x.size(1), x.size(2), code(x), stream(x));
   return pair(dx, dw, true);
@@ -265,7 +281,7 @@ PyObject* causal_conv1d_k4_backward(const Args& a) {
 PyObject* moe_router_topk_backward(const Args& a) {
   const Tensor &dw = a.t(0), &l = a.t(1), &ti = a.t(2);
   const Tensor dz = a.opt(4), dp = a.opt(5);
-  Tensor o = like(l);
+  Tensor o = like(a, 1);
   if (l.size(0))
     run(pulsar_moe_router_topk_backward, p<uint16_t>(dw), p(l), code(l), p<int64_t>(ti), a.f32(3),
                                           p<float>(dz), p<float>(dp), q(o), l.size(0), l.size(1),
@@ -288,7 +304,7 @@ PyObject* moe_dispatch_backward(const Args& a) {
 PyObject* moe_combine_backward(const Args& a) {
   const Tensor &d = a.t(0), &eo = a.t(1), &ti = a.t(2), &w = a.t(3), &ts = a.t(4);
   const int64_t N = ti.size(0), K = ti.size(1);
-  Tensor de = like(eo), dw = make(eo, {N, K}, at::kBFloat16);
+  Tensor de = like(a, 1), dw = make(eo, {N, K}, at::kBFloat16);
   run(pulsar_moe_combine_backward, p(d), p(eo), p<int64_t>(ti), p<uint16_t>(w), p<int32_t>(ts),
                                     q(de), q<uint16_t>(dw), N, eo.size(2), K, eo.size(0), eo.size(1),
                                     code(eo), stream(eo));
